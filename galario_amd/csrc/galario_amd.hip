@@ -559,7 +559,7 @@ struct SampleSetup {
     T cosPA, sinPA;
     int phase;
     T dRA2, dDec2;
-    T dRAt, dDect;   // 2 dRArot, 2 dDecrot: the phase argument in half turns (the double kernels' sincospi)
+    T dRAt, dDect;   // dRArot, dDecrot: the phase argument in turns (the double kernels' sincos_turns)
     T dRArot, dDecrot;
 };
 
@@ -584,8 +584,8 @@ SampleSetup<T> setup_sample(T PA, T dRA, T dDec) {
     s.phase = !(s.dRArot == T(0) && s.dDecrot == T(0));
     s.dRA2 = T(double(s.dRArot) * (2. * double(T(M_PI))));
     s.dDec2 = T(double(s.dDecrot) * (2. * double(T(M_PI))));
-    s.dRAt = T(2) * s.dRArot;
-    s.dDect = T(2) * s.dDecrot;
+    s.dRAt = s.dRArot;
+    s.dDect = s.dDecrot;
     return s;
 }
 
@@ -611,10 +611,28 @@ SampleArgs<T> sample_args(const cpx<T>* S, long long rs, long long cs, int nrow,
     a.dRAt = ss.dRAt;
     a.dDect = ss.dDect;
     a.inv_duv = T(1) / duv;
+    a.ext2 = INFINITY;
     a.nd = nd;
     a.u = u;
     a.v = v;
     return a;
+}
+
+// Squared extent of a dataset: rho2 in cells (<= 0: none).
+template <typename T>
+void set_extent(SampleArgs<T>& a, double rho2, double duv) {
+    a.ext2 = rho2 > 0.0 ? rho2 * duv * duv : INFINITY;
+}
+
+// The forward chi2 sample kernel on the real spectrum.
+template <typename T>
+void launch_sample_chi2(hipStream_t s, const SampleArgs<T>& a, int nb) {
+    if (nb <= SAMPLE_ONE_ROUND) {
+        hipLaunchKernelGGL((k_sample_chi2_n<T, true, 1>), dim3(nb), dim3(256), 0, s, a, nb);
+    } else {
+        hipLaunchKernelGGL((k_sample_chi2_n<T, true, SAMPLE_PPT>), dim3((nb + SAMPLE_PPT - 1) / SAMPLE_PPT), dim3(256),
+                           0, s, a, nb);
+    }
 }
 
 // chi2 of sample args `a` into chi2_d[0] (double) and, if given, chi2_t[0].
@@ -627,10 +645,11 @@ void launch_chi2(Workspace& w, hipStream_t s, SampleArgs<T> a, const T* re, cons
     a.w = wt;
     a.partials = w.part.get<double>(nb ? nb : 1);
     t_timer.mark(ST_SAMPLE, s);
-    const unsigned ng = (nb + SAMPLE_PPT - 1) / SAMPLE_PPT;
     for (int r = t_timer.reps(ST_SAMPLE); r > 0; --r) {
-        if (nb && a.H) hipLaunchKernelGGL((k_sample_chi2_n<T, true, SAMPLE_PPT>), dim3(ng), dim3(256), 0, s, a, int(nb));
-        else if (nb) hipLaunchKernelGGL((k_sample_chi2_n<T, false, SAMPLE_PPT>), dim3(ng), dim3(256), 0, s, a, int(nb));
+        if (nb && a.H) launch_sample_chi2<T>(s, a, int(nb));
+        else if (nb)
+            hipLaunchKernelGGL((k_sample_chi2_n<T, false, SAMPLE_PPT>), dim3((nb + SAMPLE_PPT - 1) / SAMPLE_PPT),
+                               dim3(256), 0, s, a, int(nb));
     }
     t_timer.mark(ST_REDUCE, s);
     hipLaunchKernelGGL((k_sum_partials<T>), dim3(1), dim3(1024), 0, s, a.partials, int(nb), chi2_d, chi2_t);
@@ -661,7 +680,7 @@ SampleArgs<T> profile_spectrum(Workspace& w, hipStream_t s, ProfileSetup<T>& ps,
         SampleArgs<T> sa = sample_args<T>(nullptr, 0, 0, N, C, T(1), duv, ss, nd, u, v);
         sa.H = H;
         sa.ldH = ldH;
-        sa.rho2 = ex.rho2;
+        set_extent(sa, ex.rho2, double(duv));
         return sa;
     }
     RowArgs<T> ra{};
@@ -1118,17 +1137,17 @@ int chi2_profile_grad_dev(void* stream, int nr, const T* I, T Rmin, T dR, T dxy,
         SampleArgs<T> sa = sample_args<T>(nullptr, 0, 0, nxy, g.C, T(1), duv, ss, nd, u, v);
         sa.H = H;
         sa.ldH = ldH;
-        sa.rho2 = ex.rho2;
+        set_extent(sa, ex.rho2, double(duv));
         sa.re = re;
         sa.im = im;
         sa.w = wt;
         sa.flag = w.flag_dev.get<unsigned>(1);
         const unsigned nb = blocks_for(size_t(nd), 256);
         double* part = w.part.get<double>(size_t(4) * (nb ? nb : 1));
-        GradArgs<T> ga{Hh, hot, part, int(nb)};
+        GradArgs<T> ga{Hh, hot, part, int(nb), int(nb), int(nb) <= GRAD_DIRECT_BLOCKS};
         t_timer.mark(ST_SAMPLE, s);
         w.Hh_zero = false;
-        if (nb) hipLaunchKernelGGL((k_sample_grad_sym<T>), dim3(nb), dim3(256), 0, s, sa, ga);
+        if (nb) hipLaunchKernelGGL((k_sample_grad_sym<T>), dim3((nb + GPT_SINGLE - 1) / GPT_SINGLE), dim3(256), 0, s, sa, ga);
         HC(hipGetLastError());
         // adjoint passes; workgroup 0 of the adjoint column pass also sums the partials into chi2 and
         // the PA, dRA, dDec gradients (the order of k_sum_partials)
@@ -1327,11 +1346,11 @@ void launch_sample_multi(int kw, int ppt, int nb, int nw, hipStream_t s, const S
 
 template <typename T, bool MIX>
 void launch_sample_grad(int win, int nb, int nw, hipStream_t s, const SampleArgs<T>& a, const BatchPtrs<T>& b) {
-    const dim3 grid(nb, nw);
+    const dim3 grid((nb + GPT_BATCH - 1) / GPT_BATCH, nw);
     switch (win) {
-        case 2048: hipLaunchKernelGGL((k_sample_grad_sym_b<T, MIX, 2048>), grid, dim3(256), 0, s, a, b); break;
-        case GWIN: hipLaunchKernelGGL((k_sample_grad_sym_b<T, MIX, GWIN>), grid, dim3(256), 0, s, a, b); break;
-        case 4096: hipLaunchKernelGGL((k_sample_grad_sym_b<T, MIX, 4096>), grid, dim3(256), 0, s, a, b); break;
+        case 2048: hipLaunchKernelGGL((k_sample_grad_sym_b<T, MIX, 2048>), grid, dim3(256), 0, s, a, b, nb); break;
+        case GWIN: hipLaunchKernelGGL((k_sample_grad_sym_b<T, MIX, GWIN>), grid, dim3(256), 0, s, a, b, nb); break;
+        case 4096: hipLaunchKernelGGL((k_sample_grad_sym_b<T, MIX, 4096>), grid, dim3(256), 0, s, a, b, nb); break;
         default: fail(GALARIO_ERR_RUNTIME, "internal: gradient window must be 2048, 3072 or 4096 cells");
     }
 }
@@ -1405,7 +1424,7 @@ void batch_enqueue(BatchPlan<T>& P, hipStream_t s, int W, const BatchShape& sh, 
                 a.im = d.im;
                 a.w = d.w;
                 a.flag = flag;
-                a.rho2 = G.ex.rho2;
+                set_extent(a, G.ex.rho2, double(d.duv));
                 a.duv_d = d.duv_d;
                 a.inv_duv_d = 1.0 / d.duv_d;
                 b.partOff = P.off[si];
@@ -1780,14 +1799,13 @@ int chi2_profile_noalloc_dev(void* stream, int nr, const T* I, T Rmin, T dR, T d
         SampleArgs<T> sa = sample_args<T>(nullptr, 0, 0, nxy, g.C, T(1), duv, ss, nd, u, v);
         sa.H = H;
         sa.ldH = g.ldH;
-        sa.rho2 = ex.rho2;
+        set_extent(sa, ex.rho2, double(duv));
         sa.re = re;
         sa.im = im;
         sa.w = wt;
         sa.partials = part;
         sa.flag = nullptr;
-        const unsigned ng = unsigned((nb + SAMPLE_PPT - 1) / SAMPLE_PPT);
-        if (nb) hipLaunchKernelGGL((k_sample_chi2_n<T, true, SAMPLE_PPT>), dim3(ng), dim3(256), 0, s, sa, int(nb));
+        if (nb) launch_sample_chi2<T>(s, sa, int(nb));
         hipLaunchKernelGGL((k_sum_partials<T>), dim3(1), dim3(1024), 0, s, part, int(nb), chi2_d,
                            static_cast<T*>(nullptr));
         HC(hipGetLastError());

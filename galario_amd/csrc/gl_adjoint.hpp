@@ -37,186 +37,305 @@ __device__ __forceinline__ void atomic_add_f64(double* p, double v) { unsafeAtom
 // sample + its adjoint: chi2 and (PA, dRA, dDec) partials per workgroup,
 // corner gradients scattered into Hh.
 //
-// Global FP64 atomics on gfx950 are resolved beyond the per-XCD L2, so many
-// atomics on one address serialise: with log-uniform baselines ~10% of all
-// points fall in the few cells around the origin.  Each workgroup therefore
-// first accumulates its corner gradients in LDS:
-//   * cells with column < GHOT and folded row < GHOT go to a GHOT x GHOT LDS
-//     tile, flushed into one of GREP replicas of that tile (by workgroup
-//     index); the adjoint column pass folds the replicas into Hh;
-//   * other cells go to an LDS window over the bounding box of the
-//     workgroup's cells when it holds at most GWIN cells (points are stored in
-//     a locality order, so it usually does), flushed with one atomic per
-//     non-zero cell; otherwise straight to Hh.
+// Global FP64 atomics on gfx950 are resolved beyond the per-XCD L2, one request per 64-byte line and wave
+// instruction, at 17 G requests/s, and atomics on one address serialise: with log-uniform
+// baselines ~10% of all points fall in the few cells around the origin.  Each workgroup
+// therefore first accumulates its corner gradients in LDS:
+//   * in a window over the bounding box of its cells when that holds at most WIN cells (points are
+//     stored in a locality order, so where they are dense it does), flushed with one atomic per
+//     non-zero cell;
+//   * otherwise in a table of the 64-byte lines of Hh that its points touch (open addressing in the
+//     same LDS), flushed with one request per line.  256 sparse points touch 200 to 500 lines with their
+//     1.9 lines each, so the table takes a third to a half off the requests: on 64 sets of parameters
+//     and datasets of 5e5 / 1.5e6 / 3e6 points at nxy = 4096 the kernel takes 0.79 / 1.6 / 2.6 ms, against
+//     0.95 / 2.1 / 3.6 ms with every corner of a sparse point sent to memory.
+// Cells with column < GHOT and folded row < GHOT do not go to Hh but to one of GREP replicas of that
+// tile (by workgroup index), which the adjoint column pass folds into Hh.
+//
+// What bounds it: those requests and, where the points are dense, vector instruction issue (about
+// 330 instructions per 64 points).  A thread takes GPT points: the bounding box, the
+// window's clearing and flush and the wave reductions are paid once per GPT points.
 // ---------------------------------------------------------------------------
 constexpr int GHOT = 16;          // hot tile: columns [0, GHOT) x folded rows [0, GHOT)
 constexpr int GREP = 32;          // replicas of the hot tile in global memory
-constexpr int GWIN = 3072;        // LDS window capacity (cells): 26 KB with the hot tile, 6 waves per SIMD
+constexpr int GWIN = 3072;        // LDS window capacity (cells): 6 workgroups per CU
                                   // (the single call's; the batched form's autotuner also tries 2048 and 4096)
 constexpr int GHOT_ELEMS = GREP * GHOT * GHOT;
-
 template <typename T>
 struct GradArgs {
     double* Hh;          // adjoint of H, same layout (h_index, ldH), zero on entry
     double* hot;         // GREP x GHOT x GHOT replicas [rep][col][row], zero on entry
-    double* partials;    // 4 streams of per-workgroup partials: chi2, dPA, ddRA, ddDec
-    int ldp;             // stride between the streams (>= number of workgroups)
+    double* partials;    // 4 streams of partials per block of 256 points: chi2, dPA, ddRA, ddDec
+    int ldp;             // stride between the streams (>= number of blocks)
+    int nblk;            // blocks of 256 points
+    int direct;          // sparse points: 1 straight to Hh, 0 through the line table
 };
 
 __device__ __forceinline__ void lds_add_f64(double* p, double v) {
     __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
+__device__ __forceinline__ double xor_sign(double x, double s) {   // x with its sign flipped where s is negative
+    return __hiloint2double(__double2hiint(x) ^ (__double2hiint(s) & int(0x80000000u)), __double2loint(x));
+}
+
+// Slot of a line in a table of NLINE keys (0xFFFFFFFF: free), entered if it is not there; -1 when eight
+// probes find no place.  Several lanes may look for the same or for colliding lines at once.
+template <int NLINE>
+__device__ __forceinline__ int line_slot(unsigned* keys, unsigned line) {
+    unsigned h = __umulhi(line * 2654435769u, unsigned(NLINE));
+    int slot = -1;
+#pragma unroll 1
+    for (int probe = 0; probe < 8 && slot < 0; ++probe) {
+        const unsigned was = atomicCAS(&keys[h], 0xFFFFFFFFu, line);
+        if (was == 0xFFFFFFFFu || was == line) slot = int(h);
+        h = h + 1 < unsigned(NLINE) ? h + 1 : 0u;
+    }
+    return slot;
+}
+
+// One point's reverse mode (all in double).
+struct GradPoint {
+    int iu, d;           // cell (SymPoint); iu = -1: nothing to add
+    double g[4];         // gradients of corners (iu, |d|), (iu, |d + 1|), (iu + 1, |d|), (iu + 1, |d + 1|)
+};
+
+// x times the sign of y (0 for y = 0)
+__device__ __forceinline__ double times_sign(double x, double y) {
+    const int one = (__double2hiint(y) & int(0x80000000u)) | 0x3FF00000;
+    return x * __hiloint2double(y == 0.0 ? 0 : one, 0);
+}
+
 // Storage T (H and the dataset streams of `a`), arithmetic P with the scalars of `sc` (P = T, sc = a:
 // galario's arithmetic in that precision; T = float, P = double: the FP32-bulk form with FP64
 // per-point arithmetic).  The reverse mode runs in double either way.  WIN: LDS window capacity
 // (cells); a larger window keeps more workgroups off the direct atomics, a smaller one leaves room
-// for more workgroups per CU.
-template <typename T, typename P, int WIN = GWIN>
+// for more workgroups per CU.  blk: workgroup, covering blocks GPT blk .. GPT blk + GPT - 1 of 256 points.
+template <typename T, typename P, int WIN, int GPT>
 __device__ __forceinline__ void sample_grad_sym_body(const SampleArgs<T>& a, const SampleArgs<P>& sc,
                                                      const GradArgs<T>& g, int blk) {
-    __shared__ double win[WIN];
-    __shared__ double hot[GHOT * GHOT];
-    __shared__ double red[4][4];
-    __shared__ int box[4][4];
+    static_assert(WIN % 512 == 0, "whole rounds of the workgroup over the window and the line table");
+    __shared__ __align__(16) double win[WIN];
+    constexpr int NLINE = WIN / 8;           // lines of the sparse points' table
+    constexpr unsigned EMPTY = 0xFFFFFFFFu;
+    __shared__ unsigned keys[NLINE];
+    __shared__ double red[3 + GPT][4];
+    __shared__ unsigned box[4][4][2];        // per wave and row of 16 lanes: packed minima
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int i = blk * 256 + tid;
-    double c2 = 0.0, gpa = 0.0, gra = 0.0, gde = 0.0;
-    double gk[4] = {0.0, 0.0, 0.0, 0.0};         // corners (fl_u, m0), (fl_u, m1), (fu1, m0), (fu1, m1)
-    int cu0 = 0, cu1 = 0, cm0 = 0, cm1 = 0;
-    bool live = false, oob = false;
-    for (int j = tid; j < GHOT * GHOT; j += 256) hot[j] = 0.0;
-    if (i < a.nd) {
-        const P u0 = P(a.u[i]), v0 = P(a.v[i]);
-        const GridPos<P> p = grid_pos<true>(sc, u0, v0);
-        oob = p.oob;
-        const P q = p.q, t = p.t;
-        const int half = a.nrow / 2;
-        cu0 = p.fl_u;
-        cu1 = p.fu1;
-        cm0 = abs(p.fl_v - half);
-        cm1 = abs(p.fv1 - half);
-        const P y0 = P(a.H[h_index(cu0, cm0, a.ldH)]), y1 = P(a.H[h_index(cu0, cm1, a.ldH)]);
-        const P y3 = P(a.H[h_index(cu1, cm0, a.ldH)]), y2 = P(a.H[h_index(cu1, cm1, a.ldH)]);
-        const P z = (t * (q * ((y0 + y2) - (y1 + y3))) + (t * (y1 - y0) + q * (y3 - y0))) + y0;
-        const P a0 = fabs(y0), a1 = fabs(y1), a2 = fabs(y2), a3 = fabs(y3);
-        P amp = a0;
-        amp += (a3 - a0) * q;
-        amp += (a1 - a0) * t;
-        amp += (((a0 - a1) + a2) - a3) * t * q;
-        const P sg = copysign(P(1), z);
+    double c2[GPT], gpa = 0.0, gra = 0.0, gde = 0.0;
+    GradPoint pt[GPT];
+    bool oob_any = false;
+    unsigned blo = 0xFFFFFFFFu, bhi = 0xFFFFFFFFu;   // packed (column pair, row) minima, and of 0xFFFF - maxima
+    // (lanes beyond the data take the last point and count nothing)
+    const int base = blk * (256 * GPT);
+    P u0[GPT], v0[GPT], ore[GPT], oim[GPT], w[GPT];
+    bool valid[GPT];
+#pragma unroll
+    for (int k = 0; k < GPT; ++k) {
+        valid[k] = base + k * 256 + tid < a.nd;
+        const unsigned i = unsigned(min(k * 256 + tid, a.nd - 1 - base)) * unsigned(sizeof(T));
+        u0[k] = P(h_at(a.u + base, i));
+        v0[k] = P(h_at(a.v + base, i));
+        ore[k] = P(h_at(a.re + base, i));
+        oim[k] = P(h_at(a.im + base, i));
+        w[k] = P(h_at(a.w + base, i));
+    }
+    SymPoint<P> p[GPT];
+    SymValues<P> y[GPT];
+#pragma unroll
+    for (int k = 0; k < GPT; ++k) {
+        p[k] = sym_position(sc, u0[k], v0[k]);
+        y[k] = sym_values<P>(a.H, a.ldH, p[k].iu, p[k].d);
+    }
+#pragma unroll
+    for (int k = 0; k < GPT; ++k) {
+        const bool oob = !p[k].in | beyond_extent(sc.ext2, u0[k], v0[k]);
+        const bool live = valid[k] & !oob;
+        oob_any |= valid[k] & oob;
         P cth = P(1), sth = P(0);
-        if (sc.phase) phase_factor(sc, p.urot, p.vrot, &sth, &cth);
-        const P V0 = copysign(amp, z);
+        if (std::is_same<P, double>::value || sc.phase) phase_factor(sc, p[k].urot, p[k].vrot, &sth, &cth);
+        const P V0 = sym_amplitude(y[k], p[k].q, p[k].t);
         const P Vre = V0 * cth, Vim = V0 * sth;
-        const P w = P(a.w[i]), ore = P(a.re[i]), oim = P(a.im[i]);
-        const P sw = sqrt(w);
-        const P cr = (Vre - ore) * sw, ci = (Vim - oim) * sw;
-        if constexpr (std::is_same<P, double>::value) c2 = cr * cr + ci * ci;
-        else c2 = double(cr) * cr + double(ci) * ci;
+        const P dre = Vre - ore[k], dim = Vim - oim[k];
+        // a point outside the grid makes every sum NaN, a lane beyond the data adds nothing
+        const double none = valid[k] ? double(NAN) : 0.0;
+        const double term = chi2_term(weight_factor(w[k]), dre, dim);
+        c2[k] = live ? term : none;
         // reverse mode in double
-        const double Gre = 2.0 * double(w) * (double(Vre) - double(ore));
-        const double Gim = 2.0 * double(w) * (double(Vim) - double(oim));
-        const double gA = double(sg) * (Gre * double(cth) + Gim * double(sth));
-        const double gth = Gim * double(Vre) - Gre * double(Vim);
-        const double dq = double(1 - t) * double(a3 - a0) + double(t) * double(a2 - a1);
-        const double dt = double(1 - q) * double(a1 - a0) + double(q) * double(a2 - a3);
-        double s_duv;
-        if constexpr (std::is_same<P, double>::value) s_duv = p.sign_u * sc.inv_duv;   // (= sign / duv exactly)
-        else s_duv = double(p.sign_u) / double(sc.duv);
-        gpa = gA * (dq * s_duv * (-double(p.vrot)) + dt * double(sc.v_origin) * s_duv * double(p.urot));
-        const double two_pi = 6.283185307179586476925286766559;
-        gra = gth * two_pi * double(u0);
-        gde = gth * two_pi * double(v0);
-        if (!oob) {
-            const auto sgn = [](P y) { return double((y > P(0)) - (y < P(0))); };
-            gk[0] = gA * (double(1 - t) * double(1 - q)) * sgn(y0);
-            gk[1] = gA * (double(t) * double(1 - q)) * sgn(y1);
-            gk[2] = gA * (double(1 - t) * double(q)) * sgn(y3);
-            gk[3] = gA * (double(t) * double(q)) * sgn(y2);
-            live = true;
-        } else {
-            c2 = gpa = gra = gde = double(NAN);
-        }
+        const double w2 = 2.0 * double(w[k]);
+        const double Gre = w2 * double(dre), Gim = w2 * double(dim);
+        const double gA = xor_sign(ffma(Gre, double(cth), Gim * double(sth)), double(V0));
+        const double gt = ffma(Gim, double(Vre), -(Gre * double(Vim)));
+        const double gth = live ? gt : none;
+        const double q = double(p[k].q), t = double(p[k].t);
+        const double y0 = double(y[k].y0), y1 = double(y[k].y1), y2 = double(y[k].y2), y3 = double(y[k].y3);
+        const double e10 = fabs(y3) - fabs(y0), e01 = fabs(y1) - fabs(y0), e11 = (fabs(y2) - fabs(y3)) - e01;
+        // A's slopes in the grid position, turned into the slope in PA (the position in cells is
+        // (urot, vrot) / duv, both negated for a folded point)
+        const double dq = ffma(t, e11, e10), dt = ffma(q, e11, e01);
+        const double gp = gA * ffma(dt, double(p[k].urot), -(dq * double(p[k].vrot)));
+        const double gps = xor_sign(gp, double(p[k].urot));
+        gpa += live ? gps : none;
+        gra = ffma(gth, double(u0[k]), gra);
+        gde = ffma(gth, double(v0[k]), gde);
+        // corners: the bilinear weights times gA, with the corner's sign (0 for a corner that is 0)
+        const double gq = gA * q, g0 = gA - gq;
+        const double k3 = gq * t, k2 = gq - k3, k1 = g0 * t, k0 = g0 - k1;
+        pt[k].iu = live ? p[k].iu : -1;
+        pt[k].d = p[k].d;
+        pt[k].g[0] = times_sign(k0, y0);
+        pt[k].g[1] = times_sign(k1, y1);
+        pt[k].g[2] = times_sign(k2, y3);
+        pt[k].g[3] = times_sign(k3, y2);
+        const int m0 = row_lo(p[k].d), m1 = row_hi(p[k].d);
+        const unsigned lo = unsigned(p[k].iu >> 1) | (unsigned(min(m0, m1)) << 16);
+        const unsigned hi = ~(unsigned((p[k].iu + 1) >> 1) | (unsigned(max(m0, m1)) << 16));
+        blo = pk_min_u16(blo, live ? lo : 0xFFFFFFFFu);
+        bhi = pk_min_u16(bhi, live ? hi : 0xFFFFFFFFu);
     }
-    if (oob && a.flag) atomicOr(a.flag, 1u);
+    if (oob_any && a.flag) atomicOr(a.flag, 1u);
     // bounding box of the workgroup's cells, columns in pairs (the window follows h_index)
-    int b0 = live ? (cu0 >> 1) : INT_MAX, b1 = live ? (cu1 >> 1) : -1;
-    int b2 = live ? min(cm0, cm1) : INT_MAX, b3 = live ? max(cm0, cm1) : -1;
-    wave_minmax2(b0, b1, b2, b3, lane);
-    if (lane == 0) {
-        box[wv][0] = b0;
-        box[wv][1] = b1;
-        box[wv][2] = b2;
-        box[wv][3] = b3;
-    }
+    const unsigned bx = row_pk_min2(blo, bhi, lane);
+    if ((lane & 15) < 2) box[wv][lane >> 4][lane & 1] = bx;
     __syncthreads();
-    const int pmin = min(min(box[0][0], box[1][0]), min(box[2][0], box[3][0]));
-    const int pmax = max(max(box[0][1], box[1][1]), max(box[2][1], box[3][1]));
-    const int mmin = min(min(box[0][2], box[1][2]), min(box[2][2], box[3][2]));
-    const int mmax = max(max(box[0][3], box[1][3]), max(box[2][3], box[3][3]));
-    const int wp = pmax - pmin + 1, wm = mmax - mmin + 1, w2 = 2 * wm;
-    const bool use_win = pmax >= 0 && wp * w2 <= WIN;      // (wp, wm <= 2^13, no overflow)
-    const int nwin = use_win ? wp * w2 : 0;
-    for (int j = tid; j < nwin; j += 256) win[j] = 0.0;
+    unsigned lo = 0xFFFFFFFFu, hi = 0xFFFFFFFFu;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        lo = pk_min_u16(lo, box[k >> 2][k & 3][0]);
+        hi = pk_min_u16(hi, box[k >> 2][k & 3][1]);
+    }
+    const bool any = lo != 0xFFFFFFFFu;   // (a live point's columns are below 2^13)
+    hi = ~hi;
+    const int pmin = int(lo & 0xFFFFu), mmin = int(lo >> 16);
+    const int wp = int(hi & 0xFFFFu) - pmin + 1, w2 = 2 * (int(hi >> 16) - mmin + 1);
+    const bool use_win = any && wp * w2 <= WIN;      // (wp, w2 <= 2^14, no overflow)
+    const int nwin = use_win ? wp * w2 : 0;          // even
+    for (int j = 2 * tid; j < (use_win ? nwin : WIN); j += 512) {
+        win[j] = 0.0;
+        win[j + 1] = 0.0;
+    }
+    double* rep = g.hot + size_t(blk % GREP) * (GHOT * GHOT);
     __syncthreads();
     if (use_win) {
-        // LDS additions, corner by corner.  Neighbouring lanes (points in locality order) often add to the
-        // same cell: lanes l and l ^ 1, then l and l ^ 2, with the same cell merge their values into the
-        // lower lane first (DPP moves), which halves to quarters the same-address LDS atomics where the
-        // points are dense.  key: window offset, or 2^30 + hot-tile offset; -1: nothing to add.
-        const int cu[4] = {cu0, cu0, cu1, cu1}, cm[4] = {cm0, cm1, cm0, cm1};
+        // LDS additions.  Neighbouring lanes (points in locality order) often lie in the same
+        // cell: lanes l and l ^ 1, then l and l ^ 2, of one cell add their four corner values into the
+        // lower lane first (DPP moves), which halves to quarters the same-address LDS atomics where
+        // the points are dense.  key: the cell, -1: nothing to add (iu = -1).
+        const int c0 = -(pmin * w2 + 2 * mmin);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const bool hotc = cu[k] < GHOT && cm[k] < GHOT;
-            int key = (live && gk[k] != 0.0)
-                          ? (hotc ? (1 << 30) + cu[k] * GHOT + cm[k]
-                                  : ((cu[k] >> 1) - pmin) * w2 + 2 * (cm[k] - mmin) + (cu[k] & 1))
-                          : -1;
-            double val = gk[k];
-            int ko = dpp_i32<DPP_XOR1>(key);
-            double vo = dpp_f64<DPP_XOR1>(val);
-            if (key >= 0 && key == ko) {
-                if (lane & 1) key = -1;
-                else val += vo;
+        for (int k = 0; k < GPT; ++k) {
+            int key = pt[k].iu < 0 ? -1 : pt[k].iu * 32768 + (pt[k].d + 8192);
+            double x0 = pt[k].g[0], x1 = pt[k].g[1], x2 = pt[k].g[2], x3 = pt[k].g[3];
+            {
+                const bool same = key == dpp_i32<DPP_XOR1>(key);
+                const double f = same ? 1.0 : 0.0;
+                x0 = ffma(dpp_f64<DPP_XOR1>(x0), f, x0);
+                x1 = ffma(dpp_f64<DPP_XOR1>(x1), f, x1);
+                x2 = ffma(dpp_f64<DPP_XOR1>(x2), f, x2);
+                x3 = ffma(dpp_f64<DPP_XOR1>(x3), f, x3);
+                key = same && (lane & 1) ? -1 : key;
             }
-            ko = dpp_i32<DPP_XOR2>(key);
-            vo = dpp_f64<DPP_XOR2>(val);
-            if (key >= 0 && key == ko) {
-                if (lane & 2) key = -1;
-                else val += vo;
+            {
+                const bool same = key == dpp_i32<DPP_XOR2>(key);
+                const double f = same ? 1.0 : 0.0;
+                x0 = ffma(dpp_f64<DPP_XOR2>(x0), f, x0);
+                x1 = ffma(dpp_f64<DPP_XOR2>(x1), f, x1);
+                x2 = ffma(dpp_f64<DPP_XOR2>(x2), f, x2);
+                x3 = ffma(dpp_f64<DPP_XOR2>(x3), f, x3);
+                key = same && (lane & 2) ? -1 : key;
             }
-            if (key >= (1 << 30)) lds_add_f64(&hot[key - (1 << 30)], val);
-            else if (key >= 0) lds_add_f64(&win[key], val);
+            if (key >= 0) {
+                const int iu = pt[k].iu, d = pt[k].d;
+                const int o0 = c0 + __mul24(iu >> 1, w2) + (iu & 1) + 2 * row_lo(d);
+                const int o2 = o0 + (iu & 1 ? w2 - 1 : 1);
+                const int dm = d >= 0 ? 2 : -2;
+                lds_add_f64(&win[o0], x0);
+                lds_add_f64(&win[o0 + dm], x1);
+                lds_add_f64(&win[o2], x2);
+                lds_add_f64(&win[o2 + dm], x3);
+            }
         }
     } else {
-        // Straight to Hh.  The FP64 atomics are served per 64-byte line and wave instruction, and
-        // a point's four corners lie in one 32-byte run of Hh when its lower column is even
-        // (h_index), so lane quads issue them together: in round r, lane l carries corner l & 3
-        // (gk order) of point (l >> 2) + 16 r of its wave.
+        // Sparse points: a table of 64-byte lines of Hh (2 columns x 4 rows, h_index), open addressing,
+        // built and flushed for one block of 256 points at a time.
+        for (int k = 0; k < GPT; ++k) {
+            GradPoint p = pt[0];          // (shadows the positions, which are done with)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int src = (lane >> 2) + 16 * r, corner = lane & 3;
-            const int c_lo = __shfl(cu0, src, 64), c_hi = __shfl(cu1, src, 64);
-            const int m_a = __shfl(cm0, src, 64), m_b = __shfl(cm1, src, 64);
-            const double g0 = __shfl(gk[0], src, 64), g1 = __shfl(gk[1], src, 64);
-            const double g2 = __shfl(gk[2], src, 64), g3 = __shfl(gk[3], src, 64);
-            const int col = (corner >> 1) ? c_hi : c_lo;
-            const int m = (corner & 1) ? m_b : m_a;
-            const double x = corner == 0 ? g0 : corner == 1 ? g1 : corner == 2 ? g2 : g3;
-            if (x != 0.0) {
-                if (col < GHOT && m < GHOT) lds_add_f64(&hot[col * GHOT + m], x);
-                else atomic_add_f64(g.Hh + h_index(col, m, a.ldH), x);
+            for (int j = 1; j < GPT; ++j)
+                if (j == k) p = pt[j];
+            for (int j = tid; j < NLINE; j += 256) keys[j] = EMPTY;
+            __syncthreads();
+            if (g.direct) {
+                if (p.iu >= 0) {
+                    const int m0 = row_lo(p.d), m1 = row_hi(p.d);
+                    const auto add = [&](int col, int m, double x) {
+                        if (x == 0.0) return;
+                        double* to = g.Hh + h_index(col, m, a.ldH);
+                        if (col < GHOT && m < GHOT) to = rep + col * GHOT + m;
+                        atomic_add_f64(to, x);
+                    };
+                    add(p.iu, m0, p.g[0]);
+                    add(p.iu, m1, p.g[1]);
+                    add(p.iu + 1, m0, p.g[2]);
+                    add(p.iu + 1, m1, p.g[3]);
+                }
+                continue;
             }
+            if (p.iu >= 0) {
+                const int m0 = row_lo(p.d), m1 = row_hi(p.d);
+                const unsigned ld4 = unsigned(a.ldH) >> 2;
+                const unsigned p0 = unsigned(p.iu >> 1) * ld4, p1 = unsigned((p.iu + 1) >> 1) * ld4;
+                const unsigned r0 = unsigned(m0 >> 2), r1 = unsigned(m1 >> 2);
+                const int e0 = 2 * (m0 & 3), e1 = 2 * (m1 & 3), o0 = p.iu & 1, o1 = o0 ^ 1;
+                const int s00 = line_slot<NLINE>(keys, p0 + r0);
+                const int s01 = r1 == r0 ? s00 : line_slot<NLINE>(keys, p0 + r1);
+                int s10 = s00, s11 = s01;
+                if (p1 != p0) {
+                    s10 = line_slot<NLINE>(keys, p1 + r0);
+                    s11 = r1 == r0 ? s10 : line_slot<NLINE>(keys, p1 + r1);
+                }
+                const auto add = [&](int slot, int e, int col, int m, double x) {
+                    if (slot >= 0) lds_add_f64(&win[8 * slot + e], x);
+                    else if (col < GHOT && m < GHOT) atomic_add_f64(rep + col * GHOT + m, x);
+                    else atomic_add_f64(g.Hh + h_index(col, m, a.ldH), x);
+                };
+                add(s00, e0 + o0, p.iu, m0, p.g[0]);
+                add(s01, e1 + o0, p.iu, m1, p.g[1]);
+                add(s10, e0 + o1, p.iu + 1, m0, p.g[2]);
+                add(s11, e1 + o1, p.iu + 1, m1, p.g[3]);
+            }
+            __syncthreads();
+            // eight lanes per line: element e of line `key` is Hh[8 key + e]; FB rounds' LDS reads together
+            const unsigned ld4 = unsigned(a.ldH) >> 2;
+            constexpr int FB = 2;
+            static_assert(8 * NLINE % (256 * FB) == 0, "whole rounds");
+            for (int j0 = tid; j0 < 8 * NLINE; j0 += 256 * FB) {
+                unsigned key[FB];
+                double x[FB];
+#pragma unroll
+                for (int h = 0; h < FB; ++h) {
+                    key[h] = keys[(j0 + 256 * h) >> 3];
+                    x[h] = win[j0 + 256 * h];
+                }
+#pragma unroll
+                for (int h = 0; h < FB; ++h) {
+                    const int j = j0 + 256 * h;
+                    if (k + 1 < GPT) win[j] = 0.0;
+                    if (key[h] != EMPTY && x[h] != 0.0) {
+                        double* to = g.Hh + size_t(key[h]) * 8 + (j & 7);
+                        if (key[h] < unsigned(GHOT / 2) * ld4) {
+                            const unsigned cp = key[h] / ld4, r = key[h] - cp * ld4;
+                            if (r < unsigned(GHOT / 4)) to = rep + (2 * cp + (j & 1)) * GHOT + 4 * r + ((j >> 1) & 3);
+                        }
+                        atomic_add_f64(to, x[h]);
+                    }
+                }
+            }
+            __syncthreads();
         }
     }
-    __syncthreads();
-    {
-        double* rep = g.hot + size_t(blk % GREP) * (GHOT * GHOT);
-        for (int j = tid; j < GHOT * GHOT; j += 256) {
-            const double x = hot[j];
-            if (x != 0.0) atomic_add_f64(rep + j, x);
-        }
+    if (use_win) {
+        __syncthreads();
         // window cell j = cp * w2 + 2 mm + (column & 1) is Hh offset ((pmin + cp) ldH + mmin) * 2 + j - cp * w2
         // (consecutive j, consecutive addresses); cp from a float reciprocal (exact after one
         // correction, j < 2^24)
@@ -227,27 +346,55 @@ __device__ __forceinline__ void sample_grad_sym_body(const SampleArgs<T>& a, con
                 int c = int(float(j) * inv_w2);
                 c += (c + 1) * w2 <= j;
                 c -= c * w2 > j;
-                atomic_add_f64(g.Hh + (size_t(pmin + c) * a.ldH + mmin) * 2 + (j - c * w2), x);
+                const int o = j - c * w2, cp = pmin + c, m = mmin + (o >> 1);
+                double* to = g.Hh + (size_t(cp) * a.ldH + mmin) * 2 + o;
+                if (cp < GHOT / 2 && m < GHOT) to = rep + (2 * cp + (o & 1)) * GHOT + m;
+                atomic_add_f64(to, x);
             }
         }
     }
-    // per-workgroup partials of chi2, dPA, ddRA, ddDec (fixed order; chi2 in the forward kernels' order,
-    // so the gradient call's chi2 equals the forward call's bit for bit)
-    c2 = wave_sum(c2);
+    // partials of chi2 per block of 256 points (the forward kernels' order, so the gradient call's chi2
+    // equals the forward call's bit for bit), of dPA, ddRA, ddDec per workgroup (the scale factors
+    // 1 / duv and 2 pi applied to the sums), stored with the first block
     wave_sum3(gpa, gra, gde, lane);
+#pragma unroll
+    for (int k = 0; k < GPT; ++k) {
+        const double x = wave_sum(c2[k]);
+        if (lane == 0) red[3 + k][wv] = x;
+    }
     if (lane == 0) {
-        red[0][wv] = c2;
-        red[1][wv] = gpa;
-        red[2][wv] = gra;
-        red[3][wv] = gde;
+        red[0][wv] = gpa;
+        red[1][wv] = gra;
+        red[2][wv] = gde;
     }
     __syncthreads();
-    if (tid < 4) g.partials[size_t(tid) * g.ldp + blk] = (red[tid][0] + red[tid][1]) + (red[tid][2] + red[tid][3]);
+    if (tid < 4 * GPT) {
+        const int st = tid & 3, k = tid >> 2, b = blk * GPT + k;
+        const int r = st == 0 ? 3 + k : st - 1;
+        double x = (red[r][0] + red[r][1]) + (red[r][2] + red[r][3]);
+        if (st == 1) {
+            if constexpr (std::is_same<P, double>::value) x *= sc.inv_duv;
+            else x /= double(sc.duv);
+        } else if (st > 1) {
+            x *= 6.283185307179586476925286766559;
+        }
+        if (st != 0 && k != 0) x = 0.0;
+        if (b < g.nblk) g.partials[size_t(st) * g.ldp + b] = x;
+    }
 }
 
+// Points per thread.  One call (1e6 points at nxy = 4096): 1, since its 3907 workgroups take two and a half
+// rounds of the chip and 1954 longer ones end with a half-empty round (77.2 against 80.2 us per gradient call);
+// the batched form: 2 (7.07 against 7.45 ms with 1 and 9.3 ms with 4, whose 180 VGPRs leave two waves per
+// SIMD, on 64 sets x 5e6 points).
+constexpr int GPT_SINGLE = 1, GPT_BATCH = 2;
+// One call with at most this many blocks of points adds its sparse points straight to Hh: the line table
+// costs such a call, which is one workgroup's latency, 1.9 us (5003 points at nxy = 512: 6.9 against
+// 5.0 us), the atomics of 8192 sparse points at four requests each about as much.
+constexpr int GRAD_DIRECT_BLOCKS = 32;
 template <typename T>
 __global__ __launch_bounds__(256) void k_sample_grad_sym(SampleArgs<T> a, GradArgs<T> g) {
-    sample_grad_sym_body<T, T>(a, a, g, blockIdx.x);
+    sample_grad_sym_body<T, T, GWIN, GPT_SINGLE>(a, a, g, blockIdx.x);
 }
 
 // Destinations of the 4 partial streams (chi2, dPA, ddRA, ddDec).

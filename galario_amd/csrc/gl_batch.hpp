@@ -26,7 +26,7 @@ struct WalkerPrm {
     T cosPA, sinPA;
     int phase;
     T dRA2, dDec2;       // 2 pi dRArot, 2 pi dDecrot
-    T dRAt, dDect;       // 2 dRArot, 2 dDecrot (the phase in half turns)
+    T dRAt, dDect;       // dRArot, dDecrot (the phase in turns)
     double tan_inc;
     // the same rotation and phase scalars in double (the FP32-bulk form's FP64 per-point arithmetic)
     double cosPAd, sinPAd, dRA2d, dDec2d, dRAtd, dDectd;
@@ -63,8 +63,8 @@ __global__ __launch_bounds__(256) void k_batch_setup(int W, const G* __restrict_
         p.phase = !(dRArot == T(0) && dDecrot == T(0));
         p.dRA2 = T(double(dRArot) * (2. * double(T(M_PI))));
         p.dDec2 = T(double(dDecrot) * (2. * double(T(M_PI))));
-        p.dRAt = T(2) * dRArot;
-        p.dDect = T(2) * dDecrot;
+        p.dRAt = dRArot;
+        p.dDect = dDecrot;
         const double PAd = double(geom[4 * i + 1]), dRAd = double(geom[4 * i + 2]), dDecd = double(geom[4 * i + 3]);
         double dRArotd = dRAd, dDecrotd = dDecd;
         p.cosPAd = 1.0;
@@ -78,8 +78,8 @@ __global__ __launch_bounds__(256) void k_batch_setup(int W, const G* __restrict_
         p.phased = !(dRArotd == 0.0 && dDecrotd == 0.0);
         p.dRA2d = dRArotd * (2. * M_PI);
         p.dDec2d = dDecrotd * (2. * M_PI);
-        p.dRAtd = 2.0 * dRArotd;
-        p.dDectd = 2.0 * dDecrotd;
+        p.dRAtd = dRArotd;
+        p.dDectd = dDecrotd;
         wp[i] = p;
     }
     if (gI && i < size_t(W) * size_t(nr)) gI[i] = 0.0;
@@ -154,7 +154,7 @@ __device__ __forceinline__ void walker_sample_args(SampleArgs<T>& a, const Batch
 }
 
 // Scalars of the FP64 per-point arithmetic for walker w on the dataset of `a` (only the fields
-// grid_pos and apply_phase_pt read).
+// sym_position and phase_factor read).
 template <typename T>
 __device__ __forceinline__ SampleArgs<double> walker_scalars_f64(const SampleArgs<T>& a, const BatchPtrs<T>& b,
                                                                  int w) {
@@ -165,7 +165,7 @@ __device__ __forceinline__ SampleArgs<double> walker_scalars_f64(const SampleArg
     sc.v_origin = double(a.v_origin);
     sc.duv = a.duv_d;
     sc.inv_duv = a.inv_duv_d;
-    sc.rho2 = a.rho2;
+    sc.ext2 = a.ext2;
     sc.rotate = p.rotate;
     sc.cosPA = p.cosPAd;
     sc.sinPA = p.sinPAd;
@@ -187,68 +187,74 @@ __device__ __forceinline__ SampleArgs<double> walker_scalars_f64(const SampleArg
 template <typename T, int KW, bool MIX = false, int PPT = 1>
 __global__ __launch_bounds__(256) void k_sample_multi_b(SampleArgs<T> a, BatchPtrs<T> b, int nw, int nblocks) {
     using P = std::conditional_t<MIX, double, T>;
-    __shared__ double red[PPT][KW][4];
+    __shared__ double red[PPT][KW][16];       // per wave and row of 16 lanes
     const int s0 = blockIdx.y * KW;
     double acc[PPT][KW];
     bool oob_any = false;
+    // (lanes beyond the data take the last point and count nothing, slots beyond the chunk the last slot)
+    const int base = blockIdx.x * (256 * PPT);
 #pragma unroll
     for (int q = 0; q < PPT; ++q) {
+        const bool valid = base + q * 256 + int(threadIdx.x) < a.nd;
+        const unsigned i = unsigned(min(q * 256 + int(threadIdx.x), a.nd - 1 - base)) * unsigned(sizeof(T));
+        P u0 = P(h_at(a.u + base, i)), v0 = P(h_at(a.v + base, i));
+        const P re = P(h_at(a.re + base, i)), im = P(h_at(a.im + base, i));
+        const P wf = weight_factor(P(h_at(a.w + base, i)));
+        const bool beyond = beyond_extent(a.ext2, u0, v0);
 #pragma unroll
-        for (int k = 0; k < KW; ++k) acc[q][k] = 0.0;
-        const int i = (blockIdx.x * PPT + q) * 256 + threadIdx.x;
-        if (i < a.nd) {
-            const P u0 = P(a.u[i]), v0 = P(a.v[i]);
-            const P re = P(a.re[i]), im = P(a.im[i]);
-            const P sw = sqrt(P(a.w[i]));
-#pragma unroll
-            for (int k = 0; k < KW; ++k) {
-                const int slot = s0 + k;
-                if (slot < nw) {
-                    SampleArgs<T> ak = a;
-                    walker_sample_args(ak, b, slot, b.w0 + slot);
-                    bool oob = false;
-                    cpx<P> V;
-                    if constexpr (MIX)
-                        V = sample_point_sym2<T, double>(ak, walker_scalars_f64(a, b, b.w0 + slot), u0, v0, oob);
-                    else
-                        V = sample_point_sym(ak, u0, v0, oob);
-                    oob_any |= oob;
-                    const P cr = (V.re - re) * sw;
-                    const P ci = (V.im - im) * sw;
-                    if constexpr (std::is_same<P, double>::value) acc[q][k] = cr * cr + ci * ci;
-                    else acc[q][k] = double(cr) * cr + double(ci) * ci;
-                }
+        for (int k = 0; k < KW; ++k) {
+            const int slot = min(s0 + k, nw - 1);
+            SampleArgs<T> ak = a;
+            walker_sample_args(ak, b, slot, b.w0 + slot);
+            bool in;
+            cpx<P> V;
+            if constexpr (MIX) {
+                const SampleArgs<double> sc = walker_scalars_f64(a, b, b.w0 + slot);
+                const SymPoint<double> p = sym_position(sc, u0, v0);
+                in = p.in;
+                V = sample_point_sym2<T, double>(ak, sc, p);
+            } else {
+                const SymPoint<T> p = sym_position(ak, u0, v0);
+                in = p.in;
+                V = sample_point_sym2<T, T>(ak, ak, p);
             }
+            const bool oob = !in | beyond;
+            oob_any |= oob & valid;
+            const double x = chi2_term(wf, V.re - re, V.im - im);
+            acc[q][k] = valid ? (oob ? double(NAN) : x) : 0.0;
+            // one walker after the other: scheduled together, eight walkers' points take 188 VGPRs (2 waves per
+            // SIMD) instead of 60, or spill
+            asm volatile("" : "+v"(u0), "+v"(v0), "+v"(acc[q][k]));
         }
     }
     if (oob_any && a.flag) atomicOr(a.flag, 1u);
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
 #pragma unroll
     for (int q = 0; q < PPT; ++q) {
-#pragma unroll
-        for (int k = 0; k < KW; ++k) {
-            const double x = wave_sum(acc[q][k]);
-            if (lane == 0) red[q][k][wv] = x;
-        }
+        const double x = joint_row_sums<KW>(acc[q], lane);
+        if ((lane & 15) < KW) red[q][lane & 15][4 * wv + (lane >> 4)] = x;
     }
     __syncthreads();
     if (threadIdx.x < PPT * KW) {
         const int q = threadIdx.x / KW, k = threadIdx.x % KW;
         const int blk = blockIdx.x * PPT + q;
+        double ws[4];                          // the waves' sums in wave_sum's order
+#pragma unroll
+        for (int w = 0; w < 4; ++w)
+            ws[w] = (red[q][k][4 * w] + red[q][k][4 * w + 1]) + (red[q][k][4 * w + 2] + red[q][k][4 * w + 3]);
         if (s0 + k < nw && blk < nblocks)
-            b.part[size_t(b.w0 + s0 + k) * 4 * b.ldPart + b.partOff + blk] =
-                (red[q][k][0] + red[q][k][1]) + (red[q][k][2] + red[q][k][3]);
+            b.part[size_t(b.w0 + s0 + k) * 4 * b.ldPart + b.partOff + blk] = (ws[0] + ws[1]) + (ws[2] + ws[3]);
     }
 }
 
 template <typename T, bool MIX = false, int WIN = GWIN>
-__global__ __launch_bounds__(256) void k_sample_grad_sym_b(SampleArgs<T> a, BatchPtrs<T> b) {
+__global__ __launch_bounds__(256) void k_sample_grad_sym_b(SampleArgs<T> a, BatchPtrs<T> b, int nblocks) {
     const int slot = blockIdx.y, w = b.w0 + slot;
     walker_sample_args(a, b, slot, w);
     double* hh = b.Hh + slot * b.sHh;
-    const GradArgs<T> g{hh, hh + b.hot_off, b.part + size_t(w) * 4 * b.ldPart + b.partOff, b.ldPart};
-    if constexpr (MIX) sample_grad_sym_body<T, double, WIN>(a, walker_scalars_f64(a, b, w), g, blockIdx.x);
-    else sample_grad_sym_body<T, T, WIN>(a, a, g, blockIdx.x);
+    const GradArgs<T> g{hh, hh + b.hot_off, b.part + size_t(w) * 4 * b.ldPart + b.partOff, b.ldPart, nblocks, 0};
+    if constexpr (MIX) sample_grad_sym_body<T, double, WIN, GPT_BATCH>(a, walker_scalars_f64(a, b, w), g, blockIdx.x);
+    else sample_grad_sym_body<T, T, WIN, GPT_BATCH>(a, a, g, blockIdx.x);
 }
 
 template <typename T, int LOG2N>

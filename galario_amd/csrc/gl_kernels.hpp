@@ -595,7 +595,7 @@ struct SampleArgs {
     T v_origin, duv;
     int rotate;  T cosPA, sinPA;
     int phase;   T dRA2, dDec2;  // 2*pi*dRArot, 2*pi*dDecrot
-    T dRAt, dDect;               // 2*dRArot, 2*dDecrot: the phase in half turns (double: sincospi)
+    T dRAt, dDect;               // dRArot, dDecrot: the phase in turns (double: sincos_turns)
     T inv_duv;                   // 1/duv (double: the grid position multiplies by it)
     int nd;
     const T* u; const T* v;
@@ -604,12 +604,13 @@ struct SampleArgs {
     const T* re; const T* im; const T* w;
     double* partials;            // MODE_CHI2: one per workgroup
     unsigned* flag;              // bit 0: a point fell outside the grid
-    double rho2;                 // > 0: squared uv extent in cells; points beyond it count as outside
+    double ext2;                 // squared uv extent in uv units, points beyond it count as outside (infinite: none)
     double duv_d, inv_duv_d;     // duv and 1/duv in double (the FP32-bulk form's FP64 per-point arithmetic)
 };
 
 // Grid coordinates of a (rotated) point; oob when it is not inside the grid
-// (or on its last row/column, where the weight beyond is zero).
+// (or on its last row/column, where the weight beyond is zero).  The general
+// complex path's form, in galario's order of operations.
 template <typename T>
 struct GridPos {
     int fl_u, fl_v, fu1, fv1;
@@ -617,11 +618,7 @@ struct GridPos {
     bool oob;
 };
 
-// RECIP (the real, even spectrum, in double): the two divisions by duv become multiplications by
-// 1/duv, within an ulp of the quotients (4e-13 cells at the grid's edge).  The interpolated
-// phase is then 0 or pi, so the sample moves by that ulp only.  The general complex path keeps
-// the divisions: galario's phase atan2(Z) amplifies a change of the position by 1/|Z|.
-template <bool RECIP = false, typename T>
+template <typename T>
 __device__ __forceinline__ GridPos<T> grid_pos(const SampleArgs<T>& a, T u0, T v0) {
     GridPos<T> g;
     g.urot = u0;
@@ -631,19 +628,9 @@ __device__ __forceinline__ GridPos<T> grid_pos(const SampleArgs<T>& a, T u0, T v
         g.vrot = u0 * a.sinPA + v0 * a.cosPA;
     }
     g.sign_u = copysign(T(1), g.urot);
-    T indu, indv;
-    if constexpr (RECIP && std::is_same<T, double>::value) {
-        indu = fabs(g.urot) * a.inv_duv;
-        indv = T(a.nrow / 2) + a.v_origin * g.sign_u * g.vrot * a.inv_duv;
-    } else {
-        indu = fabs(g.urot) / a.duv;
-        indv = T(a.nrow / 2) + a.v_origin * g.sign_u * g.vrot / a.duv;
-    }
+    const T indu = fabs(g.urot) / a.duv;
+    const T indv = T(a.nrow / 2) + a.v_origin * g.sign_u * g.vrot / a.duv;
     g.oob = !(indu <= T(a.ncol - 1) && indv >= T(0) && indv <= T(a.nrow - 1));
-    if (a.rho2 > 0.0) {   // beyond the declared extent: the spectrum there may not have been stored
-        const double du = double(indu), dv = double(indv) - double(a.nrow / 2);
-        if (du * du + dv * dv > a.rho2) g.oob = true;
-    }
     g.fl_u = g.oob ? 0 : int(floor(indu));
     g.fl_v = g.oob ? 0 : int(floor(indv));
     g.q = indu - T(g.fl_u);
@@ -653,13 +640,65 @@ __device__ __forceinline__ GridPos<T> grid_pos(const SampleArgs<T>& a, T u0, T v
     return g;
 }
 
-// e^{i theta}, theta = urot 2 pi dRArot + vrot 2 pi dDecrot.  In double as sincospi of theta / pi
-// (argument reduction by exact subtraction instead of the division by 2 pi of sincos); the angle
-// agrees to an ulp.
+// a b + c d and a b - c d: in double one product is fused into the sum (an ulp of the grid position is
+// 4e-13 cells at most); in float each operation rounds, as the reference's do.
+template <typename P>
+__device__ __forceinline__ P dot2(P a, P b, P c, P d) {
+    if constexpr (std::is_same<P, double>::value) return ffma(a, b, c * d);
+    else return a * b + c * d;
+}
+template <typename P>
+__device__ __forceinline__ P det2(P a, P b, P c, P d) {
+    if constexpr (std::is_same<P, double>::value) return ffma(a, b, -(c * d));
+    else return a * b - c * d;
+}
+
+// a b + c with the constant c in scalar registers: a vector constant would be rebuilt by two register
+// moves in front of every term of a polynomial.
+__device__ __forceinline__ double fma_const(double a, double b, double c) {
+    double r;
+    asm("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "s"(c));
+    return r;
+}
+
+// sin and cos of 2 pi x, x in turns.  f = x - (nearest integer) and then g = f - n / 4, |g| <= 1/8, n the
+// integer nearest to 4 f (rounded by the addition of 1.5 2^52, whose low word then holds n); both
+// differences are exact.  Minimax polynomials in z = g^2 (Remez; truncation error of the sine 3e-18
+// relative, of the cosine 3e-20): sin(2 pi g) = 2 pi g + g z S(z), cos(2 pi g) = 1 + z C(z).  Each result is
+// within 1.03 ulp over 2e7 arguments up to 1e3 turns, in 35 vector instructions and no branch; the
+// library's sincospi takes 72.
+__device__ __forceinline__ void sincos_turns(double x, double* s, double* c) {
+    const double big = 6755399441055744.0;   // 1.5 * 2^52
+    const double f = x - rint(x);
+    const double sh = ffma(f, 4.0, big);
+    const unsigned n = unsigned(__double2loint(sh));
+    const double g = ffma(-0.25, sh - big, f);
+    const double z = g * g;
+    double ps = ffma(z, 0.0004615925796822367 * 8192.0, -0.00737003384915244 * 2048.0);
+    ps = fma_const(ps, z, 0.08214587013039897 * 512.0);
+    ps = fma_const(ps, z, -0.5992645289748814 * 128.0);
+    ps = fma_const(ps, z, 2.5501640398740073 * 32.0);
+    ps = fma_const(ps, z, -5.16771278004996 * 8.0);
+    const double S = ffma(g, 6.28318530717958647692, (g * z) * ps);
+    double pc = ffma(z, -0.00010357788609251752 * 16384.0, 0.0019294681734144596 * 4096.0);
+    pc = fma_const(pc, z, -0.025806885879331866 * 1024.0);
+    pc = fma_const(pc, z, 0.23533063020160833 * 256.0);
+    pc = fma_const(pc, z, -1.3352627688521883 * 64.0);
+    pc = fma_const(pc, z, 4.058712126416751 * 16.0);
+    pc = fma_const(pc, z, -4.934802200544679 * 4.0);
+    const double C = ffma(z, pc, 1.0);
+    const bool odd = n & 1;
+    const double s0 = odd ? C : S, c0 = odd ? S : C;
+    const unsigned fs = (n << 30) & 0x80000000u, fc = ((n + 1) << 30) & 0x80000000u;
+    *s = __hiloint2double(int(unsigned(__double2hiint(s0)) ^ fs), __double2loint(s0));
+    *c = __hiloint2double(int(unsigned(__double2hiint(c0)) ^ fc), __double2loint(c0));
+}
+
+// e^{i theta}, theta = 2 pi (urot dRArot + vrot dDecrot).  In double from theta / 2 pi.
 template <typename T>
 __device__ __forceinline__ void phase_factor(const SampleArgs<T>& a, T urot, T vrot, T* s, T* c) {
     if constexpr (std::is_same<T, double>::value) {
-        sincospi(urot * a.dRAt + vrot * a.dDect, s, c);
+        sincos_turns(dot2(urot, a.dRAt, vrot, a.dDect), s, c);
     } else {
         fsincos(urot * a.dRA2 + vrot * a.dDec2, s, c);
     }
@@ -705,7 +744,7 @@ __device__ __forceinline__ cpx<T> sample_point(const SampleArgs<T>& a, T u0, T v
     return V;
 }
 
-// Same on the real, even spectrum H: the corners are real, Z is real, the
+// The same on the real, even spectrum H: the corners are real, Z is real, the
 // phase of galario's amplitude/phase interpolation is 0 or pi, so
 // V = (copysign(A, Z), 0) before the phase shift.
 //
@@ -713,30 +752,155 @@ __device__ __forceinline__ cpx<T> sample_point(const SampleArgs<T>& a, T u0, T v
 // while the position, interpolation and phase use the scalars of `sc` and
 // arithmetic in P.  P = T (sc = a) is galario's arithmetic in that precision;
 // T = float, P = double is the FP32-bulk form with FP64 per-point arithmetic.
-template <typename T, typename P>
-__device__ __forceinline__ cpx<P> sample_point_sym2(const SampleArgs<T>& a, const SampleArgs<P>& sc, P u0, P v0,
-                                                    bool& oob) {
-    const GridPos<P> g = grid_pos<true>(sc, u0, v0);
-    oob = g.oob;
-    const P q = g.q, t = g.t;
-    const int half = a.nrow / 2;
-    const int m0 = abs(g.fl_v - half), m1 = abs(g.fv1 - half);
-    const P y0 = P(a.H[h_index(g.fl_u, m0, a.ldH)]), y1 = P(a.H[h_index(g.fl_u, m1, a.ldH)]);
-    const P y3 = P(a.H[h_index(g.fu1, m0, a.ldH)]), y2 = P(a.H[h_index(g.fu1, m1, a.ldH)]);
-    const P z = (t * (q * ((y0 + y2) - (y1 + y3))) + (t * (y1 - y0) + q * (y3 - y0))) + y0;
-    const P a0 = fabs(y0), a1 = fabs(y1), a2 = fabs(y2), a3 = fabs(y3);
-    P amp = a0;
-    amp += (a3 - a0) * q;
-    amp += (a1 - a0) * t;
-    amp += (((a0 - a1) + a2) - a3) * t * q;
-    cpx<P> V = apply_phase_pt(sc, g, cpx<P>{copysign(amp, z), P(0)});
-    if (oob) V = cpx<P>{P(NAN), P(NAN)};
-    return V;
+//
+// The batched sample kernels issue vector instructions at 60 to 85% of the rate the chip can (nxy = 4096 and 2048;
+// 130 instructions per walker and 64 points became 105: 256 walkers x 3 datasets 2.58 to 2.11 ms), so the forms below are the ones with few instructions and no branches (a branch also
+// keeps the loads of one point behind the arithmetic of another): without a rotation the scalars are
+// cos = 1, sin = 0 (no selection per point), without offsets the phase factor of 0 is computed; the
+// real path's v_origin is 1; the extent is checked on the unrotated radius, once per point for all
+// walkers; the fraction of the position comes from one instruction; corners are 32-bit byte
+// offsets from H (H holds at most 2^28 bytes); in double the bilinear forms are nested fused products.
+// Every kernel samples through these functions, so one point gives the same bits in all of them.
+template <typename P>
+struct SymPoint {
+    int iu, d;           // cell: column, signed row (the folded rows of its corners: |d| and |d + 1|)
+    P q, t;              // position inside it
+    P urot, vrot;
+    bool in;             // inside the grid
+};
+
+// Point beyond the extent declared for the dataset (or not a number).
+template <typename P>
+__device__ __forceinline__ bool beyond_extent(double ext2, P u0, P v0) {
+    const double u = double(u0), v = double(v0);
+    return !(ffma(u, u, v * v) <= ext2);
 }
 
+// The integer part of x >= 0; 0 for x < 0 and NaN, the largest integer for x beyond it (the
+// instruction's own limits, which a C++ conversion would leave undefined).
+__device__ __forceinline__ unsigned to_u32(double x) {
+    unsigned r;
+    asm("v_cvt_u32_f64 %0, %1" : "=v"(r) : "v"(x));
+    return r;
+}
+__device__ __forceinline__ unsigned to_u32(float x) {
+    unsigned r;
+    asm("v_cvt_u32_f32 %0, %1" : "=v"(r) : "v"(x));
+    return r;
+}
+
+// A point outside the grid gets some cell inside it.
+template <typename P>
+__device__ __forceinline__ SymPoint<P> sym_position(const SampleArgs<P>& sc, P u0, P v0) {
+    SymPoint<P> p;
+    p.urot = det2(u0, sc.cosPA, v0, sc.sinPA);
+    p.vrot = dot2(u0, sc.sinPA, v0, sc.cosPA);
+    const int half = sc.nrow / 2;
+    P indu, indv;
+    if constexpr (std::is_same<P, double>::value) {
+        const double vs = __hiloint2double(
+            __double2hiint(p.vrot) ^ (__double2hiint(p.urot) & int(0x80000000u)), __double2loint(p.vrot));
+        indu = fabs(p.urot) * sc.inv_duv;
+        indv = ffma(vs, sc.inv_duv, P(half));
+        p.t = __builtin_amdgcn_fract(indv);
+    } else {
+        indu = fabs(p.urot) / sc.duv;
+        indv = P(half) + (signbit(p.urot) ? -p.vrot : p.vrot) / sc.duv;
+        p.t = __builtin_amdgcn_fractf(indv);
+    }
+    p.in = (indu <= P(sc.ncol - 1)) & (indv >= P(0)) & (indv <= P(sc.nrow - 1));
+    // (inside, both are >= 0: truncation is the floor)
+    p.iu = int(min(to_u32(indu), unsigned(half - 1)));   // (the last column: position 1 in the cell before it)
+    p.q = indu - P(p.iu);
+    p.d = int(min(to_u32(indv), unsigned(sc.nrow - 1))) - half;
+    return p;
+}
+
+// The folded rows of a cell's corners.
+__device__ __forceinline__ int row_lo(int d) { return max(d, -d); }        // |d|
+__device__ __forceinline__ int row_hi(int d) { return max(d + 1, ~d); }    // |d + 1|
+
+// H element at a byte offset (uniform base, 32-bit offset: one address register per corner)
+template <typename T>
+__device__ __forceinline__ T h_at(const T* H, unsigned bytes) {
+    return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(H) + size_t(bytes));
+}
+
+// Corner values y0 = (iu, |d|), y1 = (iu, |d + 1|), y3 = (iu + 1, |d|), y2 = (iu + 1, |d + 1|) in P.
+template <typename P>
+struct SymValues {
+    P y0, y1, y2, y3;
+};
+template <typename P, typename T>
+__device__ __forceinline__ SymValues<P> sym_values(const T* H, int ldH, int iu, int d) {
+    constexpr unsigned B = sizeof(T);
+    const unsigned ld2 = 2u * B * unsigned(ldH);                  // bytes per column pair (< 2^24)
+    const unsigned odd = unsigned(iu) & 1u;
+    const unsigned b0 = __umul24(unsigned(iu) >> 1, ld2) + odd * B;
+    const unsigned dc = odd ? ld2 - B : B;
+    const unsigned o0 = b0 + 2u * B * unsigned(row_lo(d)), o1 = b0 + 2u * B * unsigned(row_hi(d));
+    SymValues<P> y;
+    y.y0 = P(h_at(H, o0));
+    y.y1 = P(h_at(H, o1));
+    y.y3 = P(h_at(H, o0 + dc));
+    y.y2 = P(h_at(H, o1 + dc));
+    return y;
+}
+
+// copysign(A, Z): the interpolated real visibility.
+template <typename P>
+__device__ __forceinline__ P sym_amplitude(const SymValues<P>& y, P q, P t) {
+    const P a0 = fabs(y.y0), a1 = fabs(y.y1), a2 = fabs(y.y2), a3 = fabs(y.y3);
+    if constexpr (std::is_same<P, double>::value) {
+        const P z10 = y.y3 - y.y0, z01 = y.y1 - y.y0, z11 = (y.y2 - y.y3) - z01;
+        const P z = ffma(q, ffma(t, z11, z10), ffma(t, z01, y.y0));
+        const P e10 = a3 - a0, e01 = a1 - a0, e11 = (a2 - a3) - e01;
+        return copysign(ffma(q, ffma(t, e11, e10), ffma(t, e01, a0)), z);
+    } else {
+        const P z = (t * (q * ((y.y0 + y.y2) - (y.y1 + y.y3))) + (t * (y.y1 - y.y0) + q * (y.y3 - y.y0))) + y.y0;
+        P amp = a0;
+        amp += (a3 - a0) * q;
+        amp += (a1 - a0) * t;
+        amp += (((a0 - a1) + a2) - a3) * t * q;
+        return copysign(amp, z);
+    }
+}
+
+// Visibility of a point (of some cell's values where p.in is false).
+template <typename T, typename P>
+__device__ __forceinline__ cpx<P> sample_point_sym2(const SampleArgs<T>& a, const SampleArgs<P>& sc,
+                                                    const SymPoint<P>& p) {
+    const SymValues<P> y = sym_values<P>(a.H, a.ldH, p.iu, p.d);
+    P s = P(0), c = P(1);
+    if (std::is_same<P, double>::value || sc.phase) phase_factor(sc, p.urot, p.vrot, &s, &c);
+    const P V0 = sym_amplitude(y, p.q, p.t);
+    return cpx<P>{V0 * c, V0 * s};
+}
+
+// Visibility of a point on the real path; NaN and oob outside the grid or the extent.
 template <typename T>
 __device__ __forceinline__ cpx<T> sample_point_sym(const SampleArgs<T>& a, T u0, T v0, bool& oob) {
-    return sample_point_sym2<T, T>(a, a, u0, v0, oob);
+    const SymPoint<T> p = sym_position(a, u0, v0);
+    oob = !p.in | beyond_extent(a.ext2, u0, v0);
+    const cpx<T> V = sample_point_sym2<T, T>(a, a, p);
+    return oob ? cpx<T>{T(NAN), T(NAN)} : V;
+}
+
+// chi2 term w |V - O|^2 of a point.  In double from w itself (galario multiplies the residual by sqrt(w),
+// src/galario.cpp:1453-1461: NaN for a negative weight, which is kept); in float in galario's order.
+template <typename P>
+__device__ __forceinline__ P weight_factor(P w) {
+    if constexpr (std::is_same<P, double>::value) return w < P(0) ? P(NAN) : w;
+    else return sqrt(w);
+}
+template <typename P>
+__device__ __forceinline__ double chi2_term(P wf, P dre, P dim) {
+    if constexpr (std::is_same<P, double>::value) {
+        return wf * ffma(dre, dre, dim * dim);
+    } else {
+        const P cr = dre * wf, ci = dim * wf;
+        return double(cr) * cr + double(ci) * ci;
+    }
 }
 
 // Deterministic sum over a workgroup of any size <= 1024 (red: 16 doubles);
@@ -820,11 +984,7 @@ __device__ __forceinline__ void sample_body(const SampleArgs<T>& a, int blk) {
         if constexpr (MODE == MODE_VIS) {
             a.vis[a.perm ? a.perm[i] : i] = V;
         } else {
-            const T sw = sqrt(a.w[i]);
-            const T cr = (V.re - a.re[i]) * sw;
-            const T ci = (V.im - a.im[i]) * sw;
-            if constexpr (std::is_same<T, double>::value) acc = cr * cr + ci * ci;
-            else acc = double(cr) * cr + double(ci) * ci;
+            acc = chi2_term(weight_factor(a.w[i]), V.re - a.re[i], V.im - a.im[i]);
         }
     }
     if (oob && a.flag) atomicOr(a.flag, 1u);
@@ -850,9 +1010,19 @@ __device__ __forceinline__ cpx<T> multisrc_point(const SampleArgs<T>& a, int i, 
                                                  bool& oob) {
     SampleArgs<T> b = a;
     b.phase = 0;
-    const cpx<T> V0 = a.H ? sample_point_sym(b, a.u[i], a.v[i], oob) : sample_point(b, a.u[i], a.v[i], oob);
+    cpx<T> V0;
+    if (a.H) {
+        const SymPoint<T> p = sym_position(a, a.u[i], a.v[i]);
+        oob = !p.in | beyond_extent(a.ext2, a.u[i], a.v[i]);
+        V0 = cpx<T>{sym_amplitude(sym_values<T>(a.H, a.ldH, p.iu, p.d), p.q, p.t), T(0)};
+    } else {
+        V0 = sample_point(b, a.u[i], a.v[i], oob);
+    }
     T ur = a.u[i], vr = a.v[i];
-    if (a.rotate) {
+    if (a.H) {                     // the real path's rotation (sym_position)
+        ur = det2(a.u[i], a.cosPA, a.v[i], a.sinPA);
+        vr = dot2(a.u[i], a.sinPA, a.v[i], a.cosPA);
+    } else if (a.rotate) {
         ur = a.u[i] * a.cosPA - a.v[i] * a.sinPA;
         vr = a.u[i] * a.sinPA + a.v[i] * a.cosPA;
     }
@@ -869,11 +1039,12 @@ __device__ __forceinline__ cpx<T> multisrc_point(const SampleArgs<T>& a, int i, 
             SampleArgs<T> ak;          // this source's phase scalars, as setup_sample forms them
             ak.dRA2 = T(double(dRAr) * (2. * double(T(M_PI))));
             ak.dDec2 = T(double(dDecr) * (2. * double(T(M_PI))));
-            ak.dRAt = T(2) * dRAr;
-            ak.dDect = T(2) * dDecr;
+            ak.dRAt = dRAr;
+            ak.dDect = dDecr;
             T sn, cs;
             phase_factor(ak, ur, vr, &sn, &cs);
-            Vk = cpx<T>{V0.re * cs - V0.im * sn, V0.re * sn + V0.im * cs};
+            if (a.H) Vk = cpx<T>{V0.re * cs, V0.re * sn};
+            else Vk = cpx<T>{V0.re * cs - V0.im * sn, V0.re * sn + V0.im * cs};
         }
         V.re += f * Vk.re;
         V.im += f * Vk.im;
@@ -902,11 +1073,7 @@ __global__ __launch_bounds__(256) void k_sample_multisrc(SampleArgs<T> a, int ns
             if constexpr (MODE == MODE_VIS) {
                 a.vis[a.perm ? a.perm[i] : i] = V;
             } else {
-                const T sw = sqrt(a.w[i]);
-                const T cr = (V.re - a.re[i]) * sw;
-                const T ci = (V.im - a.im[i]) * sw;
-                if constexpr (std::is_same<T, double>::value) acc[q] = cr * cr + ci * ci;
-                else acc[q] = double(cr) * cr + double(ci) * ci;
+                acc[q] = chi2_term(weight_factor(a.w[i]), V.re - a.re[i], V.im - a.im[i]);
             }
         }
     }
@@ -927,10 +1094,11 @@ __global__ __launch_bounds__(256) void k_sample_multisrc(SampleArgs<T> a, int ns
 
 // chi2 with PPT blocks of 256 points per workgroup (more loads in flight per
 // wave); block q's partial is the same fixed-order sum as in k_sample.
-#ifndef GL_SAMPLE_PPT
-#define GL_SAMPLE_PPT 2
-#endif
-constexpr int SAMPLE_PPT = GL_SAMPLE_PPT;
+// PPT = 2 from more than SAMPLE_ONE_ROUND blocks on (1e6 points at nxy = 4096: 11.0 us against 11.6 with 1 and 13 with 4),
+// 1 up to there, where all workgroups of one block each are resident at once and half as many longer
+// ones would leave CUs idle (3e5 points: 0.7 us less per call).
+constexpr int SAMPLE_PPT = 2;
+constexpr int SAMPLE_ONE_ROUND = 2048;   // 256 CUs x 8 workgroups of 4 waves
 
 template <typename T, bool SYM, int PPT>
 __global__ __launch_bounds__(256) void k_sample_chi2_n(SampleArgs<T> a, int nblocks) {
@@ -938,20 +1106,27 @@ __global__ __launch_bounds__(256) void k_sample_chi2_n(SampleArgs<T> a, int nblo
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     double acc[PPT];
     bool oob_any = false;
+    // (lanes beyond the data take the last point and count nothing: no branch, so the loads of the PPT
+    // points are all in flight together)
+    const int base = blockIdx.x * (256 * PPT);
+    T u0[PPT], v0[PPT], re[PPT], im[PPT], w[PPT];
 #pragma unroll
     for (int q = 0; q < PPT; ++q) {
-        acc[q] = 0.0;
-        const int i = (blockIdx.x * PPT + q) * 256 + tid;
-        if (i < a.nd) {
-            bool oob = false;
-            const cpx<T> V = SYM ? sample_point_sym(a, a.u[i], a.v[i], oob) : sample_point(a, a.u[i], a.v[i], oob);
-            oob_any |= oob;
-            const T sw = sqrt(a.w[i]);
-            const T cr = (V.re - a.re[i]) * sw;
-            const T ci = (V.im - a.im[i]) * sw;
-            if constexpr (std::is_same<T, double>::value) acc[q] = cr * cr + ci * ci;
-            else acc[q] = double(cr) * cr + double(ci) * ci;
-        }
+        const unsigned i = unsigned(min(q * 256 + tid, a.nd - 1 - base)) * unsigned(sizeof(T));
+        u0[q] = h_at(a.u + base, i);
+        v0[q] = h_at(a.v + base, i);
+        re[q] = h_at(a.re + base, i);
+        im[q] = h_at(a.im + base, i);
+        w[q] = h_at(a.w + base, i);
+    }
+#pragma unroll
+    for (int q = 0; q < PPT; ++q) {
+        const bool valid = base + q * 256 + tid < a.nd;
+        bool oob = false;
+        const cpx<T> V = SYM ? sample_point_sym(a, u0[q], v0[q], oob) : sample_point(a, u0[q], v0[q], oob);
+        oob_any |= oob & valid;
+        const double x = chi2_term(weight_factor(w[q]), V.re - re[q], V.im - im[q]);
+        acc[q] = valid ? x : 0.0;
     }
     if (oob_any && a.flag) atomicOr(a.flag, 1u);
 #pragma unroll
@@ -1016,12 +1191,8 @@ __global__ __launch_bounds__(256) void k_chi2_terms(int nd, const T* re, const T
     const int i = blockIdx.x * 256 + threadIdx.x;
     double acc = 0.0;
     if (i < nd) {
-        const T sw = sqrt(w[i]);
         const cpx<T> V = vis[i];
-        const T cr = (V.re - re[i]) * sw;
-        const T ci = (V.im - im[i]) * sw;
-        if constexpr (std::is_same<T, double>::value) acc = cr * cr + ci * ci;
-        else acc = double(cr) * cr + double(ci) * ci;
+        acc = chi2_term(weight_factor(w[i]), V.re - re[i], V.im - im[i]);
     }
     const double b = block_sum256(acc, red);
     if (threadIdx.x == 0) a.partials[blockIdx.x] = b;
