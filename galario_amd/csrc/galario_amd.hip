@@ -1344,13 +1344,22 @@ void launch_sample_multi(int kw, int ppt, int nb, int nw, hipStream_t s, const S
     }
 }
 
+template <typename T, bool MIX, int WIN>
+void launch_sample_grad_win(int nb, int nw, hipStream_t s, const SampleArgs<T>& a, const BatchPtrs<T>& b) {
+    if (size_t(nb) * size_t(nw) <= GRAD_FEW_WORKGROUPS) {
+        hipLaunchKernelGGL((k_sample_grad_sym_b<T, MIX, WIN, 1>), dim3(nb, nw), dim3(256), 0, s, a, b, nb);
+    } else {
+        hipLaunchKernelGGL((k_sample_grad_sym_b<T, MIX, WIN, GPT_BATCH>), dim3((nb + GPT_BATCH - 1) / GPT_BATCH, nw),
+                           dim3(256), 0, s, a, b, nb);
+    }
+}
+
 template <typename T, bool MIX>
 void launch_sample_grad(int win, int nb, int nw, hipStream_t s, const SampleArgs<T>& a, const BatchPtrs<T>& b) {
-    const dim3 grid((nb + GPT_BATCH - 1) / GPT_BATCH, nw);
     switch (win) {
-        case 2048: hipLaunchKernelGGL((k_sample_grad_sym_b<T, MIX, 2048>), grid, dim3(256), 0, s, a, b, nb); break;
-        case GWIN: hipLaunchKernelGGL((k_sample_grad_sym_b<T, MIX, GWIN>), grid, dim3(256), 0, s, a, b, nb); break;
-        case 4096: hipLaunchKernelGGL((k_sample_grad_sym_b<T, MIX, 4096>), grid, dim3(256), 0, s, a, b, nb); break;
+        case 2048: launch_sample_grad_win<T, MIX, 2048>(nb, nw, s, a, b); break;
+        case GWIN: launch_sample_grad_win<T, MIX, GWIN>(nb, nw, s, a, b); break;
+        case 4096: launch_sample_grad_win<T, MIX, 4096>(nb, nw, s, a, b); break;
         default: fail(GALARIO_ERR_RUNTIME, "internal: gradient window must be 2048, 3072 or 4096 cells");
     }
 }

@@ -388,6 +388,8 @@ __device__ __forceinline__ void sample_grad_sym_body(const SampleArgs<T>& a, con
 // the batched form: 2 (7.07 against 7.45 ms with 1 and 9.3 ms with 4, whose 180 VGPRs leave two waves per
 // SIMD, on 64 sets x 5e6 points).
 constexpr int GPT_SINGLE = 1, GPT_BATCH = 2;
+// Batched launches of at most this many one-point workgroups take one point per thread too.
+constexpr size_t GRAD_FEW_WORKGROUPS = 8192;
 // One call with at most this many blocks of points adds its sparse points straight to Hh: the line table
 // costs such a call, which is one workgroup's latency, 1.9 us (5003 points at nxy = 512: 6.9 against
 // 5.0 us), the atomics of 8192 sparse points at four requests each about as much.

@@ -247,14 +247,14 @@ __global__ __launch_bounds__(256) void k_sample_multi_b(SampleArgs<T> a, BatchPt
     }
 }
 
-template <typename T, bool MIX = false, int WIN = GWIN>
+template <typename T, bool MIX, int WIN, int GPT>
 __global__ __launch_bounds__(256) void k_sample_grad_sym_b(SampleArgs<T> a, BatchPtrs<T> b, int nblocks) {
     const int slot = blockIdx.y, w = b.w0 + slot;
     walker_sample_args(a, b, slot, w);
     double* hh = b.Hh + slot * b.sHh;
     const GradArgs<T> g{hh, hh + b.hot_off, b.part + size_t(w) * 4 * b.ldPart + b.partOff, b.ldPart, nblocks, 0};
-    if constexpr (MIX) sample_grad_sym_body<T, double, WIN, GPT_BATCH>(a, walker_scalars_f64(a, b, w), g, blockIdx.x);
-    else sample_grad_sym_body<T, T, WIN, GPT_BATCH>(a, a, g, blockIdx.x);
+    if constexpr (MIX) sample_grad_sym_body<T, double, WIN, GPT>(a, walker_scalars_f64(a, b, w), g, blockIdx.x);
+    else sample_grad_sym_body<T, T, WIN, GPT>(a, a, g, blockIdx.x);
 }
 
 template <typename T, int LOG2N>
