@@ -130,13 +130,39 @@ struct DevBuf {
     }
 };
 
+// Pinned host memory, grow-only (at least 64 KB, then by powers of two); replaced only while no work uses it.
+struct PinnedBuf {
+    char* p = nullptr;
+    size_t cap = 0;
+    char* get(size_t bytes) {
+        if (bytes > cap || !p) {
+            size_t c = size_t(64) << 10;
+            while (c < bytes) c *= 2;
+            release();
+            const hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&p), c, hipHostMallocDefault);
+            if (e != hipSuccess) {
+                p = nullptr;
+                (void)hipGetLastError();
+                HC(e);
+            }
+            cap = c;
+        }
+        return p;
+    }
+    void release() {
+        if (p) (void)hipHostFree(p);
+        p = nullptr;
+        cap = 0;
+    }
+};
+
 struct Workspace {
     int device = -1;
     hipStream_t own = nullptr;    // stream of the host-pointer entry points
     hipStream_t last = nullptr;   // stream of the last call that used the buffers
     bool has_last = false;        // (the null stream is a valid `last`)
     hipEvent_t ev = nullptr;
-    DevBuf Tm, S, part, scal, flag_host, flag_dev;
+    DevBuf Tm, S, part, flag_dev, pack;
     DevBuf Hh, Th;                // gradient: adjoint half spectrum (kept zero between calls), adjoint rows
     bool Hh_zero = false;         // Hh holds zeros (cleared by the adjoint column pass)
     DevBuf chirp;                 // transform of the last chirp used (k_chirp_table) ...
@@ -144,18 +170,21 @@ struct Workspace {
     bool chirp_captured = false;  // a captured graph writes it too: rebuilt by every call
     DevBuf in[8];
     DevBuf out;
-    double* h_scal = nullptr;     // pinned: [0] result, [1] flag
-    unsigned dev_flag_dirty = 0;
+    double* h_scal = nullptr;     // pinned: [0] result, [1] flag; the host-array calls' kernels write them there
+    PinnedBuf h_in, h_out;        // packed inputs and results of a host-array call
+    bool stage_busy = false;      // work that uses them may be in flight
 
     void release() {
-        Tm.release(); S.release(); part.release(); scal.release(); Hh.release(); Th.release();
+        Tm.release(); S.release(); part.release(); pack.release(); Hh.release(); Th.release();
         Hh_zero = false;
         chirp.release();
         chirp_n = chirp_prec = 0;
         chirp_captured = false;
-        flag_host.release(); flag_dev.release(); out.release();
+        flag_dev.release(); out.release();
         for (auto& b : in) b.release();
         if (h_scal) (void)hipHostFree(h_scal);
+        h_in.release(); h_out.release();
+        stage_busy = false;
         if (ev) (void)hipEventDestroy(ev);
         if (own) (void)hipStreamDestroy(own);
         h_scal = nullptr; ev = nullptr; own = nullptr; last = nullptr; has_last = false;
@@ -213,9 +242,7 @@ Workspace& workspace(hipStream_t s, bool use_own) {
         HC(hipStreamCreateWithFlags(&n->own, hipStreamNonBlocking));
         HC(hipEventCreateWithFlags(&n->ev, hipEventDisableTiming));
         HC(hipHostMalloc(reinterpret_cast<void**>(&n->h_scal), 64, hipHostMallocDefault));
-        unsigned* fh = n->flag_host.get<unsigned>(1);
         unsigned* fd = n->flag_dev.get<unsigned>(1);
-        HC(hipMemsetAsync(fh, 0, sizeof(unsigned), n->own));
         HC(hipMemsetAsync(fd, 0, sizeof(unsigned), n->own));
         HC(hipStreamSynchronize(n->own));
         w = n.release();
@@ -772,22 +799,96 @@ void download(X* h, const X* d, size_t n, hipStream_t s) {
     if (n) HC(hipMemcpyAsync(h, d, n * sizeof(X), hipMemcpyDeviceToHost, s));
 }
 
+// Inputs and results of a host-array call.  Arrays of up to STAGE_ARRAY bytes (STAGE_BYTES in all) are packed into
+// pinned memory, which a small kernel copies to the device, STAGE_PART bytes at a time so that the copy of
+// one part runs while the next is packed: a call's six copies of a few KB cost 6 to 8 us of host
+// time each, the packed copy one launch (2013 points at nxy = 512: 78 -> 36 us a call; 40000 points
+// 127 -> 86; 2e5 points 325 -> 292).  Larger arrays go by a copy each, whose rate a copy through pinned
+// memory by one host thread does not reach (8 MB: 241 against 400 us).  The result and the out-of-grid
+// flag are written to pinned memory by the kernels themselves.
+constexpr size_t STAGE_BYTES = size_t(8) << 20, STAGE_ARRAY = size_t(2) << 20, STAGE_PART = size_t(512) << 10;
+
+struct Inputs {
+    Workspace& w;
+    hipStream_t s;
+    size_t off = 0, sent = 0;     // bytes packed, and of these on their way to the device
+    size_t cap;
+    char* dev = nullptr;
+
+    static size_t room(size_t bytes) { return (bytes + 255) & ~size_t(255); }
+
+    // total: room() of all arrays that will be added
+    Inputs(Workspace& ws, hipStream_t st, size_t total) : w(ws), s(st), cap(std::min(total, STAGE_BYTES)) {
+        if (w.stage_busy) HC(hipStreamSynchronize(s));     // a call that failed half-way
+        w.stage_busy = false;
+        w.h_scal[1] = 0.0;                                 // the out-of-grid flag
+        if (cap) {
+            w.h_in.get(cap);
+            dev = w.pack.get<char>(cap);
+        }
+    }
+    template <class X>
+    const X* add(DevBuf& b, const X* h, size_t n) {
+        const size_t bytes = n * sizeof(X);
+        if (bytes > STAGE_ARRAY || off + room(bytes) > cap) return upload(b, h, n, s);
+        char* to = w.h_in.p + off;
+        const X* d = reinterpret_cast<const X*>(dev + off);
+        if (n) std::memcpy(to, h, bytes);
+        off += room(bytes);
+        if (off - sent >= STAGE_PART) send();
+        return d;
+    }
+    // the inputs packed so far reach the device before what is launched next
+    void send() {
+        w.stage_busy = true;
+        if (off > sent) {
+            const unsigned n2 = unsigned((off - sent) / 16);
+            hipLaunchKernelGGL(k_copy16, dim3((n2 + 255) / 256), dim3(256), 0, s,
+                               reinterpret_cast<const cpx<double>*>(w.h_in.p + sent),
+                               reinterpret_cast<cpx<double>*>(dev + sent), n2);
+            HC(hipGetLastError());
+            sent = off;
+        }
+    }
+    template <class T>
+    void add_points(int nd, const T* u, const T* v, const T* re = nullptr, const T* im = nullptr,
+                    const T* wt = nullptr) {
+        const T* h[5] = {u, v, re, im, wt};
+        for (int k = 0; k < (re ? 5 : 2); ++k) points[k] = add(w.in[1 + k], h[k], size_t(nd));
+    }
+    template <class T>
+    void set_points(SampleArgs<T>& a) const {
+        a.u = static_cast<const T*>(points[0]);
+        a.v = static_cast<const T*>(points[1]);
+        a.re = static_cast<const T*>(points[2]);
+        a.im = static_cast<const T*>(points[3]);
+        a.w = static_cast<const T*>(points[4]);
+    }
+    const void* points[5] = {};
+    unsigned* flag() const { return reinterpret_cast<unsigned*>(w.h_scal + 1); }
+};
+
 // Synchronise the own stream and raise if a point fell outside the grid.
-void finish_host_call(Workspace& w, hipStream_t s, const unsigned* flag_d) {
+void finish_host_call(Workspace& w, hipStream_t s) {
     t_timer.end_call(s);
-    unsigned* hf = reinterpret_cast<unsigned*>(w.h_scal + 1);
-    HC(hipMemcpyAsync(hf, flag_d, sizeof(unsigned), hipMemcpyDeviceToHost, s));
     HC(hipStreamSynchronize(s));
-    if (*hf)
+    w.stage_busy = false;
+    if (*reinterpret_cast<volatile unsigned*>(w.h_scal + 1))
         invalid("interpolate",
                 "at least one (u, v) point falls outside the Fourier grid (|u|/duv must not exceed ncol-1 and "
                 "nrow/2 + v/duv must lie in [0, nrow-1]); increase nxy or reduce dxy");
 }
 
-unsigned* reset_host_flag(Workspace& w, hipStream_t s) {
-    unsigned* f = w.flag_host.get<unsigned>(1);
-    HC(hipMemsetAsync(f, 0, sizeof(unsigned), s));
-    return f;
+// Visibilities into the host array vis: up to STAGE_ARRAY bytes are written to pinned memory by the kernel.
+template <typename T>
+void launch_vis_host(Inputs& in, hipStream_t s, const SampleArgs<T>& sa, cpx<T>* vis) {
+    const size_t n = size_t(sa.nd), bytes = n * sizeof(cpx<T>);
+    const bool pinned = bytes <= STAGE_ARRAY;
+    cpx<T>* d = pinned ? reinterpret_cast<cpx<T>*>(in.w.h_out.get(bytes)) : in.w.out.template get<cpx<T>>(n);
+    launch_vis(s, sa, d);
+    if (!pinned) download(vis, d, n, s);
+    finish_host_call(in.w, s);
+    if (pinned && n) std::memcpy(vis, d, bytes);
 }
 
 // ------------------------------------------------------------------ main functions (host pointers)
@@ -800,16 +901,14 @@ int sample_profile_host(int nr, const T* I, T Rmin, T dR, T dxy, int nxy, T inc,
         SampleSetup<T> ss = setup_sample<T>(PA, dRA, dDec);
         Workspace& w = workspace(nullptr, true);
         hipStream_t s = w.own;
-        unsigned* flag = reset_host_flag(w, s);
-        ps.sw.I = upload(w.in[0], I, size_t(nr), s);
-        const T* du = upload(w.in[1], u, size_t(nd), s);
-        const T* dv = upload(w.in[2], v, size_t(nd), s);
-        SampleArgs<T> sa = profile_spectrum<T>(w, s, ps, ss, nxy, duv, nd, du, dv);
-        sa.flag = flag;
-        cpx<T>* dvis = w.out.get<cpx<T>>(size_t(nd));
-        launch_vis(s, sa, dvis);
-        download(reinterpret_cast<cpx<T>*>(vis), dvis, size_t(nd), s);
-        finish_host_call(w, s, flag);
+        Inputs in(w, s, Inputs::room(sizeof(T) * size_t(nr)) + 2 * Inputs::room(sizeof(T) * size_t(nd)));
+        ps.sw.I = in.add(w.in[0], I, size_t(nr));
+        in.add_points(nd, u, v);
+        in.send();
+        SampleArgs<T> sa = profile_spectrum<T>(w, s, ps, ss, nxy, duv, nd, nullptr, nullptr);
+        in.set_points(sa);
+        sa.flag = in.flag();
+        launch_vis_host(in, s, sa, reinterpret_cast<cpx<T>*>(vis));
     });
 }
 
@@ -822,19 +921,15 @@ int chi2_profile_host(int nr, const T* I, T Rmin, T dR, T dxy, int nxy, T inc, T
         SampleSetup<T> ss = setup_sample<T>(PA, dRA, dDec);
         Workspace& w = workspace(nullptr, true);
         hipStream_t s = w.own;
-        unsigned* flag = reset_host_flag(w, s);
-        ps.sw.I = upload(w.in[0], I, size_t(nr), s);
-        const T* du = upload(w.in[1], u, size_t(nd), s);
-        const T* dv = upload(w.in[2], v, size_t(nd), s);
-        const T* dre = upload(w.in[3], re, size_t(nd), s);
-        const T* dim = upload(w.in[4], im, size_t(nd), s);
-        const T* dw = upload(w.in[5], wt, size_t(nd), s);
-        SampleArgs<T> sa = profile_spectrum<T>(w, s, ps, ss, nxy, duv, nd, du, dv);
-        sa.flag = flag;
-        double* res = w.scal.get<double>(4);
-        launch_chi2<T>(w, s, sa, dre, dim, dw, res, nullptr);
-        download(w.h_scal, res, 1, s);
-        finish_host_call(w, s, flag);
+        Inputs in(w, s, Inputs::room(sizeof(T) * size_t(nr)) + 5 * Inputs::room(sizeof(T) * size_t(nd)));
+        ps.sw.I = in.add(w.in[0], I, size_t(nr));
+        in.add_points(nd, u, v, re, im, wt);
+        in.send();
+        SampleArgs<T> sa = profile_spectrum<T>(w, s, ps, ss, nxy, duv, nd, nullptr, nullptr);
+        in.set_points(sa);
+        sa.flag = in.flag();
+        launch_chi2<T>(w, s, sa, sa.re, sa.im, sa.w, w.h_scal, nullptr);
+        finish_host_call(w, s);
         *chi2 = T(w.h_scal[0]);
     });
 }
@@ -848,21 +943,19 @@ int sample_image_host(int nx, int ny, const T* image, T v_origin, T dRA, T dDec,
         SampleSetup<T> ss = setup_sample<T>(PA, dRA, dDec);
         Workspace& w = workspace(nullptr, true);
         hipStream_t s = w.own;
-        unsigned* flag = reset_host_flag(w, s);
         const int N = nx, C = N / 2 + 1;
+        Inputs in(w, s, Inputs::room(sizeof(T) * size_t(N) * N) + 2 * Inputs::room(sizeof(T) * size_t(nd)));
         RowArgs<T> ra{};
-        ra.img = upload(w.in[0], image, size_t(N) * N, s);
+        ra.img = in.add(w.in[0], image, size_t(N) * N);
         ra.ldimg = N;
-        const T* du = upload(w.in[1], u, size_t(nd), s);
-        const T* dv = upload(w.in[2], v, size_t(nd), s);
+        in.add_points(nd, u, v);
+        in.send();
         cpx<T>* S = w.S.get<cpx<T>>(size_t(C) * N);
         build_spectrum<T, SRC_IMAGE_SHIFT, OUT_COLMAJOR_SHIFT>(w, s, ra, N, N / 2, S, size_t(N));
-        SampleArgs<T> sa = sample_args<T>(S, 1, N, N, C, v_origin, duv, ss, nd, du, dv);
-        sa.flag = flag;
-        cpx<T>* dvis = w.out.get<cpx<T>>(size_t(nd));
-        launch_vis(s, sa, dvis);
-        download(reinterpret_cast<cpx<T>*>(vis), dvis, size_t(nd), s);
-        finish_host_call(w, s, flag);
+        SampleArgs<T> sa = sample_args<T>(S, 1, N, N, C, v_origin, duv, ss, nd, nullptr, nullptr);
+        in.set_points(sa);
+        sa.flag = in.flag();
+        launch_vis_host(in, s, sa, reinterpret_cast<cpx<T>*>(vis));
     });
 }
 
@@ -875,24 +968,20 @@ int chi2_image_host(int nx, int ny, const T* image, T v_origin, T dRA, T dDec, T
         SampleSetup<T> ss = setup_sample<T>(PA, dRA, dDec);
         Workspace& w = workspace(nullptr, true);
         hipStream_t s = w.own;
-        unsigned* flag = reset_host_flag(w, s);
         const int N = nx, C = N / 2 + 1;
+        Inputs in(w, s, Inputs::room(sizeof(T) * size_t(N) * N) + 5 * Inputs::room(sizeof(T) * size_t(nd)));
         RowArgs<T> ra{};
-        ra.img = upload(w.in[0], image, size_t(N) * N, s);
+        ra.img = in.add(w.in[0], image, size_t(N) * N);
         ra.ldimg = N;
-        const T* du = upload(w.in[1], u, size_t(nd), s);
-        const T* dv = upload(w.in[2], v, size_t(nd), s);
-        const T* dre = upload(w.in[3], re, size_t(nd), s);
-        const T* dim = upload(w.in[4], im, size_t(nd), s);
-        const T* dw = upload(w.in[5], wt, size_t(nd), s);
+        in.add_points(nd, u, v, re, im, wt);
+        in.send();
         cpx<T>* S = w.S.get<cpx<T>>(size_t(C) * N);
         build_spectrum<T, SRC_IMAGE_SHIFT, OUT_COLMAJOR_SHIFT>(w, s, ra, N, N / 2, S, size_t(N));
-        SampleArgs<T> sa = sample_args<T>(S, 1, N, N, C, v_origin, duv, ss, nd, du, dv);
-        sa.flag = flag;
-        double* res = w.scal.get<double>(4);
-        launch_chi2<T>(w, s, sa, dre, dim, dw, res, nullptr);
-        download(w.h_scal, res, 1, s);
-        finish_host_call(w, s, flag);
+        SampleArgs<T> sa = sample_args<T>(S, 1, N, N, C, v_origin, duv, ss, nd, nullptr, nullptr);
+        in.set_points(sa);
+        sa.flag = in.flag();
+        launch_chi2<T>(w, s, sa, sa.re, sa.im, sa.w, w.h_scal, nullptr);
+        finish_host_call(w, s);
         *chi2 = T(w.h_scal[0]);
     });
 }
@@ -1016,17 +1105,17 @@ int interpolate_host(int nrow, int ncol, const void* data, T v_origin, int nd, c
                                        std::to_string(ncol) + ")");
         Workspace& w = workspace(nullptr, true);
         hipStream_t s = w.own;
-        unsigned* flag = reset_host_flag(w, s);
+        Inputs in(w, s, 0);            // (a copy per array)
         const cpx<T>* dS = upload(w.in[0], static_cast<const cpx<T>*>(data), size_t(nrow) * ncol, s);
         const T* du = upload(w.in[1], u, size_t(nd), s);
         const T* dv = upload(w.in[2], v, size_t(nd), s);
         SampleSetup<T> ss{};   // no rotation, no phase
         SampleArgs<T> sa = sample_args<T>(dS, ncol, 1, nrow, ncol, v_origin, duv, ss, nd, du, dv);
-        sa.flag = flag;
+        sa.flag = in.flag();
         cpx<T>* dvis = w.out.get<cpx<T>>(size_t(nd));
         launch_vis(s, sa, dvis);
         download(static_cast<cpx<T>*>(vis), dvis, size_t(nd), s);
-        finish_host_call(w, s, flag);
+        finish_host_call(w, s);
     });
 }
 
@@ -1062,13 +1151,12 @@ int reduce_chi2_host(int nd, const T* re, const T* im, const void* vis, const T*
         const T* dw = upload(w.in[5], wt, size_t(nd), s);
         const cpx<T>* dvis = upload(w.out, static_cast<const cpx<T>*>(vis), size_t(nd), s);
         const unsigned nb = blocks_for(size_t(nd), 256);
-        double* res = w.scal.get<double>(4);
         SampleArgs<T> a{};
         a.partials = w.part.get<double>(nb ? nb : 1);
         if (nb) hipLaunchKernelGGL((k_chi2_terms<T>), dim3(nb), dim3(256), 0, s, nd, dre, dim, dvis, dw, a);
-        hipLaunchKernelGGL((k_sum_partials<T>), dim3(1), dim3(1024), 0, s, a.partials, int(nb), res, (T*)nullptr);
+        hipLaunchKernelGGL((k_sum_partials<T>), dim3(1), dim3(1024), 0, s, a.partials, int(nb), w.h_scal,
+                           (T*)nullptr);
         HC(hipGetLastError());
-        download(w.h_scal, res, 1, s);
         HC(hipStreamSynchronize(s));
         *chi2 = T(w.h_scal[0]);
     });

@@ -193,7 +193,7 @@ __device__ __forceinline__ void sample_grad_sym_body(const SampleArgs<T>& a, con
         blo = pk_min_u16(blo, live ? lo : 0xFFFFFFFFu);
         bhi = pk_min_u16(bhi, live ? hi : 0xFFFFFFFFu);
     }
-    if (oob_any && a.flag) atomicOr(a.flag, 1u);
+    if (oob_any && a.flag) raise_flag(a.flag);
     // bounding box of the workgroup's cells, columns in pairs (the window follows h_index)
     const unsigned bx = row_pk_min2(blo, bhi, lane);
     if ((lane & 15) < 2) box[wv][lane >> 4][lane & 1] = bx;

@@ -227,7 +227,7 @@ __global__ __launch_bounds__(256) void k_sample_multi_b(SampleArgs<T> a, BatchPt
             asm volatile("" : "+v"(u0), "+v"(v0), "+v"(acc[q][k]));
         }
     }
-    if (oob_any && a.flag) atomicOr(a.flag, 1u);
+    if (oob_any && a.flag) raise_flag(a.flag);
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
 #pragma unroll
     for (int q = 0; q < PPT; ++q) {

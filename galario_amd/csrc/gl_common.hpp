@@ -176,4 +176,9 @@ __device__ __forceinline__ unsigned row_pk_min2(unsigned lo, unsigned hi, int la
     return pk_min_u16(k, unsigned(dpp_i32<DPP_ROW_ROR8>(int(k))));
 }
 
+// Marks that a point fell outside the grid (device memory, or pinned host memory for the host-array calls).
+__device__ __forceinline__ void raise_flag(unsigned* flag) {
+    __hip_atomic_store(flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 }  // namespace gl

@@ -1106,7 +1106,7 @@ __device__ __forceinline__ void sample_body(const SampleArgs<T>& a, int blk) {
             acc = chi2_term(weight_factor(a.w[i]), V.re - a.re[i], V.im - a.im[i]);
         }
     }
-    if (oob && a.flag) atomicOr(a.flag, 1u);
+    if (oob && a.flag) raise_flag(a.flag);
     if constexpr (MODE == MODE_CHI2) {
         const double b = block_sum256(acc, red);
         if (threadIdx.x == 0) a.partials[blk] = b;
@@ -1196,7 +1196,7 @@ __global__ __launch_bounds__(256) void k_sample_multisrc(SampleArgs<T> a, int ns
             }
         }
     }
-    if (oob_any && a.flag) atomicOr(a.flag, 1u);
+    if (oob_any && a.flag) raise_flag(a.flag);
     if constexpr (MODE == MODE_CHI2) {
 #pragma unroll
         for (int q = 0; q < PPT; ++q) {
@@ -1247,7 +1247,7 @@ __global__ __launch_bounds__(256) void k_sample_chi2_n(SampleArgs<T> a, int nblo
         const double x = chi2_term(weight_factor(w[q]), V.re - re[q], V.im - im[q]);
         acc[q] = valid ? x : 0.0;
     }
-    if (oob_any && a.flag) atomicOr(a.flag, 1u);
+    if (oob_any && a.flag) raise_flag(a.flag);
 #pragma unroll
     for (int q = 0; q < PPT; ++q) {
         const double x = wave_sum(acc[q]);
@@ -1321,6 +1321,13 @@ __global__ __launch_bounds__(256) void k_chi2_terms(int nd, const T* re, const T
 __global__ __launch_bounds__(256) void k_fill_zero(double* p, size_t n) {
     const size_t i = size_t(blockIdx.x) * 256 + threadIdx.x;
     if (i < n) p[i] = 0.0;
+}
+
+// Copies n2 16-byte words (the host-array calls' packed inputs, read over the bus from pinned memory).
+__global__ __launch_bounds__(256) void k_copy16(const cpx<double>* __restrict__ in, cpx<double>* __restrict__ out,
+                                                unsigned n2) {
+    const unsigned i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n2) out[i] = in[i];
 }
 
 // Quadrant swap of the N x N real image held in rows of ld reals
