@@ -79,6 +79,11 @@ __device__ __forceinline__ double xor_sign(double x, double s) {   // x with its
     return __hiloint2double(__double2hiint(x) ^ (__double2hiint(s) & int(0x80000000u)), __double2loint(x));
 }
 
+// The same at a byte offset below 2^32 from a uniform base (Hh holds at most 2^29 bytes).
+__device__ __forceinline__ void atomic_add_at(double* base, unsigned bytes, double v) {
+    atomic_add_f64(reinterpret_cast<double*>(reinterpret_cast<char*>(base) + size_t(bytes)), v);
+}
+
 // Slot of a line in a table of NLINE keys (0xFFFFFFFF: free), entered if it is not there; -1 when eight
 // probes find no place.  Several lanes may look for the same or for colliding lines at once.
 template <int NLINE>
@@ -119,8 +124,8 @@ __device__ __forceinline__ void sample_grad_sym_body(const SampleArgs<T>& a, con
     constexpr int NLINE = WIN / 8;           // lines of the sparse points' table
     constexpr unsigned EMPTY = 0xFFFFFFFFu;
     __shared__ unsigned keys[NLINE];
-    __shared__ double red[3 + GPT][4];
-    __shared__ unsigned box[4][4][2];        // per wave and row of 16 lanes: packed minima
+    __shared__ double red[3 + GPT][16];      // per wave and row of 16 lanes
+    __shared__ unsigned box[32];             // likewise: packed minima, lo and hi in turn
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     double c2[GPT], gpa = 0.0, gra = 0.0, gde = 0.0;
     GradPoint pt[GPT];
@@ -196,24 +201,23 @@ __device__ __forceinline__ void sample_grad_sym_body(const SampleArgs<T>& a, con
     if (oob_any && a.flag) raise_flag(a.flag);
     // bounding box of the workgroup's cells, columns in pairs (the window follows h_index)
     const unsigned bx = row_pk_min2(blo, bhi, lane);
-    if ((lane & 15) < 2) box[wv][lane >> 4][lane & 1] = bx;
+    if ((lane & 15) < 2) box[8 * wv + 2 * (lane >> 4) + (lane & 1)] = bx;
     __syncthreads();
-    unsigned lo = 0xFFFFFFFFu, hi = 0xFFFFFFFFu;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-        lo = pk_min_u16(lo, box[k >> 2][k & 3][0]);
-        hi = pk_min_u16(hi, box[k >> 2][k & 3][1]);
-    }
-    const bool any = lo != 0xFFFFFFFFu;   // (a live point's columns are below 2^13)
-    hi = ~hi;
-    const int pmin = int(lo & 0xFFFFu), mmin = int(lo >> 16);
-    const int wp = int(hi & 0xFFFFu) - pmin + 1, w2 = 2 * (int(hi >> 16) - mmin + 1);
+    // the minima over the rows of all waves, as scalars: what follows from them takes no vector instructions
+    unsigned kb = box[lane & 31];
+    kb = pk_min_u16(kb, unsigned(dpp_i32<DPP_XOR2>(int(kb))));
+    kb = pk_min_u16(kb, unsigned(dpp_i32<DPP_ROW_ROR4>(int(kb))));
+    kb = pk_min_u16(kb, unsigned(dpp_i32<DPP_ROW_ROR8>(int(kb))));
+    const unsigned l0 = unsigned(__builtin_amdgcn_readlane(int(kb), 0)), l1 = unsigned(__builtin_amdgcn_readlane(int(kb), 16));
+    const unsigned h0 = unsigned(__builtin_amdgcn_readlane(int(kb), 1)), h1 = unsigned(__builtin_amdgcn_readlane(int(kb), 17));
+    const int pmin = int(min(l0 & 0xFFFFu, l1 & 0xFFFFu)), mmin = int(min(l0 >> 16, l1 >> 16));
+    const int pmax = 0xFFFF - int(min(h0 & 0xFFFFu, h1 & 0xFFFFu)), mmax = 0xFFFF - int(min(h0 >> 16, h1 >> 16));
+    const bool any = pmin <= pmax;                   // (no live point: 0xFFFF and 0)
+    const int wp = pmax - pmin + 1, w2 = 2 * (mmax - mmin + 1);
     const bool use_win = any && wp * w2 <= WIN;      // (wp, w2 <= 2^14, no overflow)
     const int nwin = use_win ? wp * w2 : 0;          // even
-    for (int j = 2 * tid; j < (use_win ? nwin : WIN); j += 512) {
-        win[j] = 0.0;
-        win[j + 1] = 0.0;
-    }
+    for (int j = 2 * tid; j < (use_win ? nwin : WIN); j += 512)
+        *reinterpret_cast<cpx<double>*>(&win[j]) = cpx<double>{0.0, 0.0};
     double* rep = g.hot + size_t(blk % GREP) * (GHOT * GHOT);
     __syncthreads();
     if (use_win) {
@@ -305,29 +309,33 @@ __device__ __forceinline__ void sample_grad_sym_body(const SampleArgs<T>& a, con
                 add(s11, e1 + o1, p.iu + 1, m1, p.g[3]);
             }
             __syncthreads();
-            // eight lanes per line: element e of line `key` is Hh[8 key + e]; FB rounds' LDS reads together
+            // eight lanes per line: element e of line `key` is Hh[8 key + e] (a line with a non-zero element has
+            // a key); FB rounds' LDS reads together, more than which cost registers (4: 7.5 against 7.07 ms)
             const unsigned ld4 = unsigned(a.ldH) >> 2;
             constexpr int FB = 2;
             static_assert(8 * NLINE % (256 * FB) == 0, "whole rounds");
+#pragma unroll 1
             for (int j0 = tid; j0 < 8 * NLINE; j0 += 256 * FB) {
                 unsigned key[FB];
                 double x[FB];
 #pragma unroll
                 for (int h = 0; h < FB; ++h) {
-                    key[h] = keys[(j0 + 256 * h) >> 3];
+                    key[h] = keys[(j0 >> 3) + 32 * h];
                     x[h] = win[j0 + 256 * h];
                 }
 #pragma unroll
                 for (int h = 0; h < FB; ++h) {
-                    const int j = j0 + 256 * h;
-                    if (k + 1 < GPT) win[j] = 0.0;
-                    if (key[h] != EMPTY && x[h] != 0.0) {
-                        double* to = g.Hh + size_t(key[h]) * 8 + (j & 7);
+                    if (k + 1 < GPT) win[j0 + 256 * h] = 0.0;
+                    if (x[h] != 0.0) {
+                        const unsigned e = unsigned(tid) & 7u;
                         if (key[h] < unsigned(GHOT / 2) * ld4) {
                             const unsigned cp = key[h] / ld4, r = key[h] - cp * ld4;
-                            if (r < unsigned(GHOT / 4)) to = rep + (2 * cp + (j & 1)) * GHOT + 4 * r + ((j >> 1) & 3);
+                            if (r < unsigned(GHOT / 4)) {
+                                atomic_add_f64(rep + (2 * cp + (e & 1)) * GHOT + 4 * r + (e >> 1), x[h]);
+                                continue;
+                            }
                         }
-                        atomic_add_f64(to, x[h]);
+                        atomic_add_at(g.Hh, (8u * key[h] + e) * 8u, x[h]);
                     }
                 }
             }
@@ -347,31 +355,31 @@ __device__ __forceinline__ void sample_grad_sym_body(const SampleArgs<T>& a, con
                 c += (c + 1) * w2 <= j;
                 c -= c * w2 > j;
                 const int o = j - c * w2, cp = pmin + c, m = mmin + (o >> 1);
-                double* to = g.Hh + (size_t(cp) * a.ldH + mmin) * 2 + o;
-                if (cp < GHOT / 2 && m < GHOT) to = rep + (2 * cp + (o & 1)) * GHOT + m;
-                atomic_add_f64(to, x);
+                if (cp < GHOT / 2 && m < GHOT) atomic_add_f64(rep + (2 * cp + (o & 1)) * GHOT + m, x);
+                else atomic_add_at(g.Hh, unsigned(2 * (cp * a.ldH + mmin) + o) * 8u, x);
             }
         }
     }
     // partials of chi2 per block of 256 points (the forward kernels' order, so the gradient call's chi2
     // equals the forward call's bit for bit), of dPA, ddRA, ddDec per workgroup (the scale factors
     // 1 / duv and 2 pi applied to the sums), stored with the first block
-    wave_sum3(gpa, gra, gde, lane);
+    const int row = 4 * wv + (lane >> 4);
+    const double sums[4] = {c2[0], gpa, gra, gde};
+    const double sum = joint_row_sums<4>(sums, lane);
+    if ((lane & 15) < 4) red[lane & 3][row] = sum;
 #pragma unroll
-    for (int k = 0; k < GPT; ++k) {
-        const double x = wave_sum(c2[k]);
-        if (lane == 0) red[3 + k][wv] = x;
-    }
-    if (lane == 0) {
-        red[0][wv] = gpa;
-        red[1][wv] = gra;
-        red[2][wv] = gde;
+    for (int k = 1; k < GPT; ++k) {
+        const double y = row_sum(c2[k]);
+        if ((lane & 15) == 0) red[3 + k][row] = y;
     }
     __syncthreads();
     if (tid < 4 * GPT) {
         const int st = tid & 3, k = tid >> 2, b = blk * GPT + k;
-        const int r = st == 0 ? 3 + k : st - 1;
-        double x = (red[r][0] + red[r][1]) + (red[r][2] + red[r][3]);
+        const double* r = red[st == 0 && k > 0 ? 3 + k : st];
+        double ws[4];                          // the waves' sums in wave_sum's order
+#pragma unroll
+        for (int w = 0; w < 4; ++w) ws[w] = (r[4 * w] + r[4 * w + 1]) + (r[4 * w + 2] + r[4 * w + 3]);
+        double x = (ws[0] + ws[1]) + (ws[2] + ws[3]);
         if (st == 1) {
             if constexpr (std::is_same<P, double>::value) x *= sc.inv_duv;
             else x /= double(sc.duv);

@@ -137,28 +137,6 @@ __device__ __forceinline__ double joint_row_sums(const double (&a)[K], int lane)
     }
 }
 
-// Three wave64 sums at once, in a fixed order of their own (not wave_sum's); all 64 lanes active,
-// results in every lane.  The lanes trade halves of the vector: after the pair step even lanes carry
-// the pair sums of (a, b) and odd lanes those of (c, 0), after the quad step lane l carries one
-// quad sum (l mod 4 = 0: a, 1: c, 2: b, 3: 0); then rows of 16 by rotations by 4 and 8 (lanes 4
-// apart carry the same sum) and the rows by two shuffles.  About half the instructions of three
-// wave_sum calls.
-__device__ __forceinline__ void wave_sum3(double& a, double& b, double& c, int lane) {
-    const bool o1 = lane & 1, o2 = lane & 2;
-    double k0 = o1 ? c : a, k1 = o1 ? 0.0 : b;
-    k0 += dpp_f64<DPP_XOR1>(o1 ? a : c);
-    k1 += dpp_f64<DPP_XOR1>(o1 ? b : 0.0);
-    double k = o2 ? k1 : k0;
-    k += dpp_f64<DPP_XOR2>(o2 ? k0 : k1);
-    k += dpp_f64<DPP_ROW_ROR4>(k);
-    k += dpp_f64<DPP_ROW_ROR8>(k);
-    k += __shfl_xor(k, 16, 64);
-    k += __shfl_xor(k, 32, 64);
-    a = lane_f64(k, 0);
-    c = lane_f64(k, 1);
-    b = lane_f64(k, 2);
-}
-
 // Two 16-bit numbers in one register (lo | hi << 16), and their elementwise unsigned minimum.
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ unsigned pk_min_u16(unsigned a, unsigned b) {
