@@ -581,6 +581,24 @@ SymGeom sym_geom(int L, int N, int rmax) {
     return g;
 }
 
+// Column pairs {2p, 2p + 1} within the store radius sqrt(rc2) (stored_rows), of the first npair; all of them
+// without a radius.  The passes launch a workgroup for these only: grids sized by galario's
+// get_image_size keep 0.4 of the columns.  Fewer than N/4 pairs leave column N/2 out.
+inline int active_pairs(int npair, double rc2) {
+    if (!(rc2 > 0.0)) return npair;
+    const double p = std::floor(std::sqrt(rc2)) / 2.0 + 1.0;
+    return p < double(npair) ? int(p) : npair;
+}
+
+// Workgroups of the column pass: whole rounds of the 8 XCDs (xcd_column).
+inline int colpass_blocks(int N, double rc2) { return 8 * ((active_pairs(N / 4, rc2) + 7) / 8); }
+
+// Frequencies of the row spectra (rows of C) that the column pass reads, in whole 64-byte blocks of ts_index.
+inline int ts_columns(int C, double rc2) {
+    const int n = active_pairs((C + 1) / 2, rc2);
+    return std::min(C, (2 * n + 3) & ~3);
+}
+
 // Real, even half spectrum H of a swept profile (see k_rowpass_sym); returns
 // false when the workgroup FFT does not cover N (the caller then uses the
 // general complex path).  zero/nzero: doubles the row pass clears (gradient
@@ -595,12 +613,13 @@ bool build_spectrum_sym(Workspace& w, hipStream_t s, const SweepPrm<T>& sw, int 
     T* Ts = w.Tm.get<T>(size_t(2 * g.pairs_r) * g.ldT);      // rows 0..nrows-1 and a padding row
     T* H = w.S.get<T>(size_t(g.C + 1) * g.ldH);
     const cpx<T>* tw = twiddles<T>(N);
-    SymRowArgs<T> ra{sw, N, g.Rs, g.nrows, g.ldT, tw, Ts, zero, nzero, zero1};
+    SymRowArgs<T> ra{sw, N, g.Rs, g.nrows, g.ldT, tw, Ts, zero, nzero, zero1, ts_columns(g.C, rc2)};
     SymColArgs<T> ca{Ts, N, g.Rs, g.ldT, tw, H, g.ldH, rc2, residue_fits(L, g.Rs) ? twiddles<T>(512) : nullptr};
     t_timer.mark(ST_ROW, s);
     for (int r = t_timer.reps(ST_ROW); r > 0; --r) launch_rowpass_sym<T>(L, g.pairs_r, s, ra);
     t_timer.mark(ST_COL, s);
-    for (int r = t_timer.reps(ST_COL); r > 0; --r) launch_colpass_sym<T>(L, N / 4, s, ca);   // N/4 pairs + column N/2
+    for (int r = t_timer.reps(ST_COL); r > 0; --r)
+        launch_colpass_sym<T>(L, colpass_blocks(N, rc2), s, ca);
     HC(hipGetLastError());
     *H_out = H;
     *ldH_out = g.ldH;
@@ -1312,7 +1331,8 @@ int chi2_profile_grad_dev(void* stream, int nr, const T* I, T Rmin, T dR, T dxy,
         T* Th = w.Th.get<T>(size_t(g.nrows) * ldTh);
         const cpx<T>* tw = twiddles<T>(nxy);
         const Dst4 dst{{chi2_d, grad_geom + 1, grad_geom + 2, grad_geom + 3}};
-        const int nfft = 8 * ((g.pairs_c + 7) / 8);
+        const int apairs = active_pairs(g.pairs_c, ex.rc2);
+        const int nfft = 8 * ((apairs + 7) / 8);
         AdjColArgs<T> aca{Hh,   hot,  g.ldH, nxy,  g.Rs,    tw,
                           Th,   ldTh, part,  int(nb), dst, nfft,
                           ex.rc2, residue_fits(L, g.Rs) ? twiddles<T>(512) : nullptr};
@@ -1321,7 +1341,8 @@ int chi2_profile_grad_dev(void* stream, int nr, const T* I, T Rmin, T dR, T dxy,
         HC(hipGetLastError());
         w.Hh_zero = true;
         AdjRowArgs<T> ara{ps.sw,  Th,        ldTh,     nxy, g.Rs, g.nrows, tw, std::tan(double(inc)),
-                          grad_I, grad_geom, aca.tw512};   // tw512 set: the residue form where it fits
+                          grad_I, grad_geom, aca.tw512,     // tw512 set: the residue form where it fits
+                          std::min(g.C, 2 * apairs)};
         t_timer.mark(ST_ADJROW, s);
         launch_adjrow_sym<T>(L, g.pairs_r, s, ara);
         HC(hipGetLastError());
@@ -1553,12 +1574,14 @@ void batch_enqueue(BatchPlan<T>& P, hipStream_t s, int W, const BatchShape& sh, 
             const SymGeom& g = G.g;
             const int L = g.L;
             const cpx<T>* tw = twiddles<T>(G.N);
-            SymRowArgs<T> ra{G.sw, G.N, g.Rs, g.nrows, g.ldT, tw, nullptr, nullptr, 0, nullptr};
+            SymRowArgs<T> ra{G.sw, G.N, g.Rs, g.nrows, g.ldT, tw, nullptr, nullptr, 0, nullptr,
+                               ts_columns(g.C, G.ex.rc2)};
             SymColArgs<T> ca{nullptr, G.N, g.Rs,     g.ldT,
                              tw,      nullptr, g.ldH, G.ex.rc2,
                              residue_fits(L, g.Rs) ? twiddles<T>(512) : nullptr};
-            const int cblocks = G.N / 4;                      // column pairs 0..N/2-1, column N/2 inside
-            const int ablocks = 8 * ((g.pairs_c + 7) / 8);    // adjoint: (C+1)/2 pairs
+            const int cblocks = colpass_blocks(G.N, G.ex.rc2);   // column pairs 0..N/2-1, column N/2 inside
+            const int apairs = active_pairs(g.pairs_c, G.ex.rc2);
+            const int ablocks = 8 * ((apairs + 7) / 8);          // adjoint: (C+1)/2 pairs
 #define GL_CALL(LL) \
     hipLaunchKernelGGL((k_rowpass_sym_b<T, LL>), dim3(g.pairs_r, nw), dim3(FftShape<LL>::NT), 0, s, ra, b)
             GL_L_SWITCH(T, GL_CALL)
@@ -1608,7 +1631,8 @@ void batch_enqueue(BatchPlan<T>& P, hipStream_t s, int W, const BatchShape& sh, 
                 AdjColArgs<T> aca{nullptr, nullptr, g.ldH, G.N, g.Rs, tw, nullptr, 0, nullptr, 0, Dst4{}, ablocks,
                                   G.ex.rc2};
                 aca.ldTh = int(P.sTh / size_t(g.nrows));
-                AdjRowArgs<T> ara{G.sw, nullptr, aca.ldTh, G.N, g.Rs, g.nrows, tw, 0.0, nullptr, nullptr};
+                AdjRowArgs<T> ara{G.sw, nullptr, aca.ldTh, G.N,     g.Rs,    g.nrows,
+                                  tw,   0.0,     nullptr,  nullptr, nullptr, std::min(g.C, 2 * apairs)};
 #define GL_CALL(LL)                                                                                              \
     hipLaunchKernelGGL((k_adjcol_sym_b<T, LL>), dim3(ablocks, nw), dim3(FftShape<LL>::NT), 0, s, aca, b);        \
     hipLaunchKernelGGL((k_adjrow_sym_b<T, LL>), dim3(g.pairs_r, nw), dim3(FftShape<LL>::NT), 0, s, ara, b)
@@ -1957,11 +1981,12 @@ int chi2_profile_noalloc_dev(void* stream, int nr, const T* I, T Rmin, T dR, T d
         const Extent ex = uv_extent<T>(uvmax, double(duv));
         ps.sw.I = I;
         hipStream_t s = static_cast<hipStream_t>(stream);
-        const SymRowArgs<T> ra{ps.sw, nxy, g.Rs, g.nrows, g.ldT, tw, Ts, nullptr, 0, nullptr};
+        const SymRowArgs<T> ra{ps.sw, nxy,     g.Rs, g.nrows, g.ldT, tw, Ts,
+                               nullptr, 0, nullptr, ts_columns(g.C, ex.rc2)};
         const SymColArgs<T> ca{Ts, nxy, g.Rs, g.ldT, tw, H, g.ldH, ex.rc2,
                                residue_fits(L, g.Rs) ? twiddles_built<T>(dev, 512) : nullptr};
         launch_rowpass_sym<T>(L, g.pairs_r, s, ra);
-        launch_colpass_sym<T>(L, nxy / 4, s, ca);
+        launch_colpass_sym<T>(L, colpass_blocks(nxy, ex.rc2), s, ca);
         SampleArgs<T> sa = sample_args<T>(nullptr, 0, 0, nxy, g.C, T(1), duv, ss, nd, u, v);
         sa.H = H;
         sa.ldH = g.ldH;

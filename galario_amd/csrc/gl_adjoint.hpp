@@ -520,14 +520,7 @@ __device__ __forceinline__ void adjcol_sym_body(const AdjColArgs<T>& a, int blk,
     // rows the sample kernel can have touched (column lb: no more); beyond them Hh, and the
     // replicas of the hot tile, hold zeros
     const int kc = stored_rows(a.rc2, la, N);
-    if (kc < 0) {                      // no sample reaches these columns: their adjoint rows are zero
-        for (int m = tid; m <= a.Rs; m += NT) {
-            T* o = a.Th + size_t(m) * a.ldTh + la;
-            o[0] = T(0);
-            if (has_b) o[1] = T(0);
-        }
-        return;
-    }
+    if (kc < 0) return;                // (the adjoint row pass reads no frequency of these columns)
     __shared__ double hs[2][GHOT];
     if (hot_cols) {
         fold_hot<NT>(a.hot, la, hs);
@@ -609,14 +602,7 @@ __device__ __forceinline__ void adjcol_sub_body(const AdjColArgs<T>& a, int blk)
     cpx<double>* hab = reinterpret_cast<cpx<double>*>(a.Hh + h_index(la, 0, a.ldH));   // columns la, lb
     const bool hot_cols = la < GHOT;   // GHOT is even: lb < GHOT too
     const int kc = stored_rows(a.rc2, la, N);
-    if (kc < 0) {                      // no sample reaches these columns: their adjoint rows are zero
-        for (int m = tid; m <= a.Rs; m += NT) {
-            T* o = a.Th + size_t(m) * a.ldTh + la;
-            o[0] = T(0);
-            if (has_b) o[1] = T(0);
-        }
-        return;
-    }
+    if (kc < 0) return;                // (the adjoint row pass reads no frequency of these columns)
     // rows 0..kc of the pair (+ the hot tile's replicas), each read by one thread and then cleared
     __shared__ double hs[2][GHOT];
     if (hot_cols) {
@@ -713,6 +699,7 @@ struct AdjRowArgs {
     double* gI;          // nr, zeroed by the forward row pass
     double* ginc;        // 1, zeroed by the forward row pass
     const cpx<T>* tw512; // W_512^e table (k_adjrow_sub)
+    int ncol;            // frequencies 0..ncol-1 of Th were written; beyond them it is zero
 };
 
 // dchi2/d(pixel value) = gz: accumulate into dI (workgroup-local copy in LDS)
@@ -785,6 +772,7 @@ __device__ __forceinline__ void adjrow_sym_body(const AdjRowArgs<T>& a, int blk)
     cpx<T> v[E];
     F::run(v, lds, tid, N / 2, a.tw, [&](int k) -> cpx<T> {
         const int l = k <= N / 2 ? k : N - k;
+        if (l >= a.ncol) return cpx<T>{T(0), T(0)};
         const T wk = T(ext_weight(k, N));
         return cpx<T>{wk * ra[l], hb ? wk * rb[l] : T(0)};
     }, a.Rs < NT);        // pixels j <= Rs' only
@@ -859,8 +847,8 @@ __device__ __forceinline__ void adjrow_sub_body(const AdjRowArgs<T>& a, int blk)
 #pragma unroll
     for (int q = 0; q < PER; ++q) {
         const int p = tid + q * NT;
-        xb[q] = (hb && p < C) ? rb[p] : T(0);
-        if (p < C) stg[p + (p >> 3)] = ra[p];
+        xb[q] = (hb && p < a.ncol) ? rb[p] : T(0);
+        if (p < C) stg[p + (p >> 3)] = p < a.ncol ? ra[p] : T(0);
     }
     __syncthreads();
     cpx<T> v[8];

@@ -328,8 +328,8 @@ struct BlockFft {
     // Full transform.  load(n) returns input element n; it is called only for
     // n in [0, Rs) U [N-Rs, N) (zeros elsewhere).  lds: LDS_ELEMS reals.  On
     // return v[r] holds X[tid + r*N/E] (only0: v[0] = X[tid] only), and every
-    // thread has finished reading LDS.
-    template <typename Loader>
+    // thread has finished reading LDS.  LOADS_LDS: load reads that same LDS.
+    template <bool LOADS_LDS = false, typename Loader>
     static __device__ __forceinline__ void run(cpx<T> (&v)[E], T* lds, int tid, int Rs,
                                                const cpx<T>* __restrict__ tw, Loader&& load, bool only0 = false) {
         constexpr int R0 = E;            // first pass is radix E, one butterfly per thread
@@ -350,6 +350,7 @@ struct BlockFft {
             }
             dft<R0, INV>(v);
         }
+        if constexpr (LOADS_LDS) __syncthreads();
         rest<1>(v, lds, tid, tw, only0);
     }
 
