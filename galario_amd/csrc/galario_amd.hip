@@ -354,6 +354,14 @@ inline bool residue_fits(int L, int Rs) { return L >= 10 && L <= 13 && Rs <= RES
         default: fail(GALARIO_ERR_RUNTIME, "internal: no residue kernel for this size"); \
     }
 
+// Whether all workgroups of a full column transform fit on the 256 CUs at once with both parts of the
+// exchange in LDS (2 * LDS_ELEMS reals of the CU's 160 KB).
+template <typename T>
+inline bool few_blocks(int L, int blocks) {
+    const size_t n = size_t(1) << L, bytes = 2 * sizeof(T) * (n + n / 16);
+    return size_t(blocks) <= 256 * ((size_t(160) << 10) / (bytes + 1024));
+}
+
 template <typename T>
 void launch_rowpass_sym(int L, int blocks, hipStream_t s, const SymRowArgs<T>& a) {
 #define GL_CALL(LL) hipLaunchKernelGGL((k_rowpass_sym<T, LL>), dim3(blocks), dim3(FftShape<LL>::NT), 0, s, a)
@@ -369,6 +377,12 @@ void launch_colpass_sym(int L, int blocks, hipStream_t s, const SymColArgs<T>& a
 #undef GL_CALL
         return;
     }
+    if (few_blocks<T>(L, blocks)) {
+#define GL_CALL(LL) hipLaunchKernelGGL((k_colpass_sym_few<T, LL>), dim3(blocks), dim3(FftShape<LL>::NT), 0, s, a)
+        GL_L_SWITCH(T, GL_CALL)
+#undef GL_CALL
+        return;
+    }
 #define GL_CALL(LL) hipLaunchKernelGGL((k_colpass_sym<T, LL>), dim3(blocks), dim3(FftShape<LL>::NT), 0, s, a)
     GL_L_SWITCH(T, GL_CALL)
 #undef GL_CALL
@@ -379,6 +393,12 @@ void launch_adjcol_sym(int L, int blocks, hipStream_t s, const AdjColArgs<T>& a)
     if (residue_fits(L, a.Rs)) {
 #define GL_CALL(LL) hipLaunchKernelGGL((k_adjcol_sub<T, LL>), dim3(blocks), dim3(ResidueShape<LL>::NT), 0, s, a)
         GL_RESIDUE_SWITCH(GL_CALL)
+#undef GL_CALL
+        return;
+    }
+    if (few_blocks<T>(L, blocks)) {
+#define GL_CALL(LL) hipLaunchKernelGGL((k_adjcol_sym_few<T, LL>), dim3(blocks), dim3(FftShape<LL>::NT), 0, s, a)
+        GL_L_SWITCH(T, GL_CALL)
 #undef GL_CALL
         return;
     }

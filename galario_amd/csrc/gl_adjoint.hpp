@@ -496,14 +496,14 @@ __device__ __forceinline__ void fold_hot(double* hot, int la, double (*hs)[GHOT]
 
 // PARTIALS: workgroups blk >= nfft sum the sample kernel's partial streams
 // (the batched form sums them in its own reduction kernel).
-template <typename T, int LOG2N, bool PARTIALS = true>
+template <typename T, int LOG2N, bool PARTIALS = true, bool SPLIT = true>
 __device__ __forceinline__ void adjcol_sym_body(const AdjColArgs<T>& a, int blk, int nblk) {
     using S = FftShape<LOG2N>;
-    using F = BlockFft<T, LOG2N, false>;
+    using F = BlockFft<T, LOG2N, false, SPLIT>;
     constexpr int N = S::N, NT = S::NT, E = S::E;
     constexpr int C = N / 2 + 1;
     constexpr int NPAIR = (C + 1) / 2;
-    __shared__ T lds[S::LDS_ELEMS];
+    __shared__ T lds[F::LDS_REALS];
     if (PARTIALS && blk >= a.nfft) {        // extra workgroups: the partial sums of the sample kernel
         const int j = blk - a.nfft;
         __shared__ double red16[16];
@@ -555,6 +555,12 @@ __device__ __forceinline__ void adjcol_sym_body(const AdjColArgs<T>& a, int blk,
 template <typename T, int LOG2N>
 __global__ __launch_bounds__(FftShape<LOG2N>::NT) void k_adjcol_sym(AdjColArgs<T> a) {
     adjcol_sym_body<T, LOG2N>(a, blockIdx.x, gridDim.x);
+}
+
+// Few workgroups: as k_colpass_sym_few.
+template <typename T, int LOG2N>
+__global__ __launch_bounds__(FftShape<LOG2N>::NT) void k_adjcol_sym_few(AdjColArgs<T> a) {
+    adjcol_sym_body<T, LOG2N, true, false>(a, blockIdx.x, gridDim.x);
 }
 
 // Residue form of the adjoint column pass (N >= 1024, profile within 255 pixels: Rs' <= 256; the single

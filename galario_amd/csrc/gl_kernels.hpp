@@ -549,13 +549,13 @@ __device__ __forceinline__ void colpass_nyquist(const SymColArgs<T>& a, int blk)
     }
 }
 
-template <typename T, int LOG2N>
+template <typename T, int LOG2N, bool SPLIT = true>
 __device__ __forceinline__ void colpass_sym_body(const SymColArgs<T>& a, int blk, int nblk) {
     using S = FftShape<LOG2N>;
-    using F = BlockFft<T, LOG2N, false>;
+    using F = BlockFft<T, LOG2N, false, SPLIT>;
     constexpr int N = S::N, NT = S::NT, E = S::E;
     constexpr int NPAIR = N / 4;                  // pairs of columns 0..N/2-1; column N/2 separately
-    __shared__ T lds[S::LDS_ELEMS];
+    __shared__ T lds[F::LDS_REALS];
     const int pair = xcd_column(blk, nblk);
     if (pair >= NPAIR) return;
     const int la = 2 * pair;
@@ -702,6 +702,12 @@ template <typename T, int LOG2N>
 __global__ __launch_bounds__(FftShape<LOG2N>::NT) __attribute__((amdgpu_waves_per_eu(4))) void k_colpass_sym(
     SymColArgs<T> a) {
     colpass_sym_body<T, LOG2N>(a, blockIdx.x, gridDim.x);
+}
+
+// Few workgroups: both parts per LDS round trip (half the barriers, twice the LDS), no register cap.
+template <typename T, int LOG2N>
+__global__ __launch_bounds__(FftShape<LOG2N>::NT) void k_colpass_sym_few(SymColArgs<T> a) {
+    colpass_sym_body<T, LOG2N, false>(a, blockIdx.x, gridDim.x);
 }
 
 // ---------------------------------------------------------------------------
