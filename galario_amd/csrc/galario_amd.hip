@@ -1567,6 +1567,20 @@ struct BatchShape {
     int chunk, kw, ppt, win;
 };
 
+// Walkers of a grid processed together in the forward form when a plan has several grids: at most `chunk`, and no more
+// than whose half spectra the 256 MB MALL about holds (a power of two, at least 8), since the samples then
+// read them from there.  256 walkers, nxy = 2048 and 1e6 points: 1.48 ms with 32, 1.54 with 128; nxy = 1024 and
+// 2e5 points, whose 128 spectra fit: 0.39 with 128, 0.53 with 32.  (With one grid the timed choice is that grid's own; the
+// gradient form, bound by its atomics, takes the largest chunk.)
+template <typename T>
+int group_chunk(const BatchPlan<T>& P, const BatchGroup<T>& G, int chunk, bool grad) {
+    if (grad || P.groups.size() < 2) return chunk;
+    const size_t bytes = sizeof(T) * size_t(G.g.C + 1) * size_t(G.g.ldH);
+    int c = 8;
+    while (size_t(2 * c) * bytes <= (size_t(288) << 20)) c *= 2;
+    return std::min(c, chunk);
+}
+
 template <typename T>
 void batch_enqueue(BatchPlan<T>& P, hipStream_t s, int W, const BatchShape& sh, int mode) {
     const int nr = P.nr, chunk = sh.chunk;
@@ -1587,10 +1601,11 @@ void batch_enqueue(BatchPlan<T>& P, hipStream_t s, int W, const BatchShape& sh, 
                            grad ? static_cast<double*>(P.ggeom.p) : nullptr);
     BatchPtrs<T> b = batch_ptrs(P, grad);
     unsigned* flag = static_cast<unsigned*>(P.flag.p);
-    for (int w0 = 0; w0 < W; w0 += chunk) {
-        const int nw = std::min(chunk, W - w0);
-        b.w0 = w0;
-        for (const BatchGroup<T>& G : P.groups) {
+    for (const BatchGroup<T>& G : P.groups) {
+        const int gchunk = group_chunk(P, G, chunk, grad);
+        for (int w0 = 0; w0 < W; w0 += gchunk) {
+            const int nw = std::min(gchunk, W - w0);
+            b.w0 = w0;
             const SymGeom& g = G.g;
             const int L = g.L;
             const cpx<T>* tw = twiddles<T>(G.N);
@@ -1806,10 +1821,10 @@ template <typename T>
 void batch_tune(BatchPlan<T>& P, hipStream_t s, int W, int mode, typename BatchPlan<T>::Exec& run) {
     const bool grad = mode & MODE_GRAD;
     const int cmax = P.max_chunk(grad, W);
-    std::vector<int> cand;
-    for (int c = 1; c < cmax; c *= 2) cand.push_back(c);
-    cand.push_back(cmax);
-    BatchShape best{cand.back(), 4, run.tile_fixed ? run.ppt : 1, run.tile_fixed ? run.win : GWIN};
+    std::vector<int> cand{cmax};                     // largest first
+    for (int c = cmax - 1; c > 0; --c)
+        if (!(c & (c - 1))) cand.push_back(c);
+    BatchShape best{cand.front(), 4, run.tile_fixed ? run.ppt : 1, run.tile_fixed ? run.win : GWIN};
     float tbest = 0.f;
     for (int c : cand) {
         BatchShape t = best;
@@ -1819,6 +1834,9 @@ void batch_tune(BatchPlan<T>& P, hipStream_t s, int W, int mode, typename BatchP
             tbest = ms;
             best.chunk = c;
         }
+        // chunks too small to fill the chip only get slower with every halving (up to twice the best time
+        // and more): 256 walkers x 3 datasets spend 176 ms in this search with them, 80 without
+        if (ms > 1.25f * tbest) break;
     }
     auto try_shape = [&](BatchShape t) {
         const float ms = batch_time(P, s, W, t, mode);
