@@ -690,7 +690,10 @@ __device__ __forceinline__ void colpass_sub_body(const SymColArgs<T>& a, int pai
 
 template <typename T, int LOG2N>
 __global__ __launch_bounds__(ResidueShape<LOG2N>::NT) void k_colpass_sub(SymColArgs<T> a) {
-    colpass_sub_body<T, LOG2N>(a, xcd_column(blockIdx.x, gridDim.x));
+    // rows of more than 64 KB (nxy = 8192 in double) pass through LDS in halves: 74 KB would leave two workgroups
+    // per CU (67.0 -> 60.6 us per forward call, 1e6 points; at 4096 the halves cost 0.8 us)
+    constexpr bool HALVES = size_t(ResidueShape<LOG2N>::N / 2) * sizeof(cpx<T>) >= 65536;
+    colpass_sub_body<T, LOG2N, HALVES>(a, xcd_column(blockIdx.x, gridDim.x));
 }
 
 // At most 128 VGPRs (4 waves per SIMD): one call's N/4 workgroups then all fit
