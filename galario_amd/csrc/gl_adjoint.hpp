@@ -230,6 +230,13 @@ __device__ __forceinline__ void sample_grad_sym_body(const SampleArgs<T>& a, con
         for (int k = 0; k < GPT; ++k) {
             int key = pt[k].iu < 0 ? -1 : pt[k].iu * 32768 + (pt[k].d + 8192);
             double x0 = pt[k].g[0], x1 = pt[k].g[1], x2 = pt[k].g[2], x3 = pt[k].g[3];
+            // (a lane with nothing to add may hold a NaN, which a factor of 0 would pass on)
+            if (__ballot(key < 0) != 0) {
+                x0 = key < 0 ? 0.0 : x0;
+                x1 = key < 0 ? 0.0 : x1;
+                x2 = key < 0 ? 0.0 : x2;
+                x3 = key < 0 ? 0.0 : x3;
+            }
             {
                 const bool same = key == dpp_i32<DPP_XOR1>(key);
                 const double f = same ? 1.0 : 0.0;
