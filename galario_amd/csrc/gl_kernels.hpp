@@ -934,7 +934,8 @@ __device__ __forceinline__ SymPoint<P> sym_position(const SampleArgs<P>& sc, P u
         const double vs = __hiloint2double(
             __double2hiint(p.vrot) ^ (__double2hiint(p.urot) & int(0x80000000u)), __double2loint(p.vrot));
         indu = fabs(p.urot) * sc.inv_duv;
-        indv = ffma(vs, sc.inv_duv, P(half));
+        // (rounded twice: a fused one puts points on the first row a last bit outside the grid)
+        indv = vs * sc.inv_duv + P(half);
         p.t = __builtin_amdgcn_fract(indv);
     } else {
         indu = fabs(p.urot) / sc.duv;

@@ -187,6 +187,22 @@ def test_grids_of_one_plan():
                 assert abs(per[k, j].item() - one) <= 1e-12 * abs(one)
 
 
+@pytest.mark.parametrize('N', [128, 1024])
+def test_grid_edge(N):
+    """A point on the last column, and on the first and last rows that have a cell, against points just inside."""
+    import galario_amd.double as gD
+    I, dR = profile()
+    duv = 1 / (N * DXY)
+    h = N // 2
+    u = np.array([h, h, 3.25, 3.25]) * duv
+    v = np.array([0.0, 5.5, (h - 1) * (1 - 1e-15), -h]) * duv
+    inside = np.array([1 - 1e-13, 1 - 1e-13, 1.0, 1.0]), np.array([1.0, 1.0, 1 - 1e-13, 1 - 1e-13])
+    a = gD.sampleProfile(I, RMIN, dR, N, DXY, u, v, inc=0.3, check_central_pixel=False)
+    b = gD.sampleProfile(I, RMIN, dR, N, DXY, u * inside[0], v * inside[1], inc=0.3, check_central_pixel=False)
+    assert np.isfinite(a).all()
+    assert (np.abs(a - b) <= 1e-9 * np.abs(b).max()).all(), (a, b)
+
+
 @pytest.mark.parametrize('offset', [0.0, 1e-9, 0.03 * O.ARCSEC, 40 * O.ARCSEC, 3.0])
 def test_phase(offset):
     """Offsets from none to many turns across the uv plane: exp(2 pi i (u dRA + v dDec)) in long double."""
