@@ -166,7 +166,7 @@ struct Workspace {
     DevBuf Hh, Th;                // gradient: adjoint half spectrum (kept zero between calls), adjoint rows
     bool Hh_zero = false;         // Hh holds zeros (cleared by the adjoint column pass)
     DevBuf chirp;                 // transform of the last chirp used (k_chirp_table) ...
-    int chirp_n = 0, chirp_prec = 0;   // ... for this N and precision (0: none)
+    int chirp_n = 0;              // ... for this N (0: none)
     bool chirp_captured = false;  // a captured graph writes it too: rebuilt by every call
     DevBuf in[8];
     DevBuf out;
@@ -178,7 +178,7 @@ struct Workspace {
         Tm.release(); S.release(); part.release(); pack.release(); Hh.release(); Th.release();
         Hh_zero = false;
         chirp.release();
-        chirp_n = chirp_prec = 0;
+        chirp_n = 0;
         chirp_captured = false;
         flag_dev.release(); out.release();
         for (auto& b : in) b.release();
@@ -454,61 +454,49 @@ void launch_colpass(int L, int blocks, hipStream_t s, const ColArgs<T>& a) {
     }
 }
 
-// log2 of the power of two M >= 2N - 1 of the chirp transform, -1 where the direct sums serve: N up to 64
+// log2 of the power of two M >= 2N - 1 of the chirp transform, -1 where the direct sums serve: float, N up to 64
 // (which they do in less time than the chirp transform's longer path) or M beyond the largest transform.
 template <typename T>
 int chirp_log2(int N) {
-    if (N <= 64) return -1;
+    if (sizeof(T) == 4 || N <= 64) return -1;
     int L = 7;
     while (L <= max_fast_log2<T>() && (1 << L) < 2 * N - 1) ++L;
     return L <= max_fast_log2<T>() ? L : -1;
 }
 
 // Tables of the chirp transform of size N = a.N.  B is kept in the thread's workspace, whose calls run in order,
-// and rebuilt (in double where the transform exists in double) when N or the precision changes.
-template <typename T>
-ChirpArgs<T> chirp_tables(Workspace& w, hipStream_t s, int N, int L) {
-    const bool in_double = L <= max_fast_log2<double>();
-    const int prec = int(sizeof(T));
-    cpx<T>* B = w.chirp.get<cpx<T>>(size_t(1) << L);
+// and rebuilt when N changes.
+ChirpArgs<double> chirp_tables(Workspace& w, hipStream_t s, int N, int L) {
+    cpx<double>* B = w.chirp.get<cpx<double>>(size_t(1) << L);
     if (s) {
         hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
         HC(hipStreamIsCapturing(s, &st));
         if (st != hipStreamCaptureStatusNone) w.chirp_captured = true;
     }
-    if (w.chirp_captured || w.chirp_n != N || w.chirp_prec != prec) {
+    const cpx<double>*tw2n = twiddles<double>(2 * N), *twm = twiddles<double>(1 << L);
+    if (w.chirp_captured || w.chirp_n != N) {
         w.chirp_n = 0;
-        if (in_double) {
-            const cpx<double>*tw2n = twiddles<double>(2 * N), *twm = twiddles<double>(1 << L);
-            switch (L) {
-#define GL_CHIRP(LL) \
-    case LL: hipLaunchKernelGGL((k_chirp_table<double, T, LL>), dim3(1), dim3(FftShape<LL>::NT), 0, s, N, tw2n, twm, B); break;
-                GL_CHIRP(7) GL_CHIRP(8) GL_CHIRP(9) GL_CHIRP(10) GL_CHIRP(11) GL_CHIRP(12) GL_CHIRP(13)
-#undef GL_CHIRP
-                default: fail(GALARIO_ERR_RUNTIME, "internal: no chirp table for this size");
-            }
-        } else if constexpr (sizeof(T) == 4) {
-            hipLaunchKernelGGL((k_chirp_table<float, float, 14>), dim3(1), dim3(FftShape<14>::NT), 0, s, N,
-                               twiddles<float>(2 * N), twiddles<float>(1 << 14), B);
-        }
+#define GL_CALL(LL) \
+    hipLaunchKernelGGL((k_chirp_table<double, LL>), dim3(1), dim3(FftShape<LL>::NT), 0, s, N, tw2n, twm, B)
+        GL_L_SWITCH(double, GL_CALL)
+#undef GL_CALL
         HC(hipGetLastError());
         w.chirp_n = N;
-        w.chirp_prec = prec;
     }
-    return ChirpArgs<T>{twiddles<T>(2 * N), twiddles<T>(1 << L), B};
+    return ChirpArgs<double>{tw2n, twm, B};
 }
 
-template <typename T, int SRC>
-void launch_rowpass_chirp(int L, int pairs, hipStream_t s, const RowArgs<T>& a, const ChirpArgs<T>& c) {
-#define GL_CALL(LL) hipLaunchKernelGGL((k_rowpass_chirp<T, LL, SRC>), dim3(pairs), dim3(FftShape<LL>::NT), 0, s, a, c)
-    GL_L_SWITCH(T, GL_CALL)
+template <int SRC>
+void launch_rowpass_chirp(int L, int pairs, hipStream_t s, const RowArgs<double>& a, const ChirpArgs<double>& c) {
+#define GL_CALL(LL) hipLaunchKernelGGL((k_rowpass_chirp<double, LL, SRC>), dim3(pairs), dim3(FftShape<LL>::NT), 0, s, a, c)
+    GL_L_SWITCH(double, GL_CALL)
 #undef GL_CALL
 }
 
-template <typename T, int OUT>
-void launch_colpass_chirp(int L, int blocks, hipStream_t s, const ColArgs<T>& a, const ChirpArgs<T>& c) {
-#define GL_CALL(LL) hipLaunchKernelGGL((k_colpass_chirp<T, LL, OUT>), dim3(blocks), dim3(FftShape<LL>::NT), 0, s, a, c)
-    GL_L_SWITCH(T, GL_CALL)
+template <int OUT>
+void launch_colpass_chirp(int L, int blocks, hipStream_t s, const ColArgs<double>& a, const ChirpArgs<double>& c) {
+#define GL_CALL(LL) hipLaunchKernelGGL((k_colpass_chirp<double, LL, OUT>), dim3(blocks), dim3(FftShape<LL>::NT), 0, s, a, c)
+    GL_L_SWITCH(double, GL_CALL)
 #undef GL_CALL
 }
 
@@ -536,16 +524,30 @@ cpx<T>* build_spectrum(Workspace& w, hipStream_t s, RowArgs<T> ra, int N, int Rs
     const int L = fast_log2<T>(N), LM = L > 0 ? -1 : chirp_log2<T>(N);
     if (LM < 0) ra.tw = ca.tw = twiddles<T>(N);
     if (LM > 0) {
-        const ChirpArgs<T> c = chirp_tables<T>(w, s, N, LM);
-        t_timer.mark(ST_ROW, s);
-        launch_rowpass_chirp<T, SRC>(LM, Rs, s, ra, c);
-        t_timer.mark(ST_COL, s);
-        launch_colpass_chirp<T, OUT>(LM, 8 * ((C + 7) / 8), s, ca, c);
+        if constexpr (sizeof(T) == 8) {
+            const ChirpArgs<T> c = chirp_tables(w, s, N, LM);
+            t_timer.mark(ST_ROW, s);
+            launch_rowpass_chirp<SRC>(LM, Rs, s, ra, c);
+            t_timer.mark(ST_COL, s);
+            launch_colpass_chirp<OUT>(LM, 8 * ((C + 7) / 8), s, ca, c);
+        }
     } else if (L > 0) {
         t_timer.mark(ST_ROW, s);
         launch_rowpass<T, SRC>(L, Rs, s, ra);
         t_timer.mark(ST_COL, s);
         launch_colpass<T, OUT>(L, 8 * ((C + 7) / 8), s, ca);
+    } else if (sizeof(T) == 4 && N <= DFT_TILED_MAX) {
+        if constexpr (sizeof(T) == 4) {
+            const size_t lds = sizeof(cpx<T>) * size_t(N);
+            allow_lds(k_rowdft_tiled<SRC>, lds);
+            allow_lds(k_coldft_tiled<OUT>, lds);
+            t_timer.mark(ST_ROW, s);
+            hipLaunchKernelGGL((k_rowdft_tiled<SRC>), dim3((2 * Rs + DFT_LINES - 1) / DFT_LINES, (C + DFT_FREQS - 1) / DFT_FREQS),
+                               dim3(256), lds, s, ra);
+            t_timer.mark(ST_COL, s);
+            hipLaunchKernelGGL((k_coldft_tiled<OUT>), dim3((C + DFT_LINES - 1) / DFT_LINES, (N + DFT_FREQS - 1) / DFT_FREQS),
+                               dim3(256), lds, s, ca);
+        }
     } else {
         const size_t lds_row = sizeof(T) * size_t(2 * Rs);
         if (lds_row > 160 * 1024) fail(GALARIO_ERR_INVALID, "Error in fft: image size not supported");

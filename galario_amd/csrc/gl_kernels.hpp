@@ -215,32 +215,32 @@ __global__ __launch_bounds__(FftShape<LOG2N>::NT) void k_colpass(ColArgs<T> a) {
 }
 
 // ---------------------------------------------------------------------------
-// other even N: Bluestein's chirp transform.  With c[n] = exp(-i pi n^2 / N),
+// other even N in double: Bluestein's chirp transform.  With c[n] = exp(-i pi n^2 / N),
 //   X[k] = c[k] sum_n (x[n] c[n]) conj(c[k - n]),
 // a convolution that a cyclic one of M >= 2N - 1 points holds: transform of x c (M points, a power of two,
 // BlockFft), times the transform B of conj(c) (k_chirp_table, scaled by 1/M), transform back, times c.
-// Two M-point transforms per row pair or column instead of N^2 products: N = 1000 in float (rows and columns
-// of an image) takes 30 us where direct sums took 900.  Chirp indices n^2 mod 2N are exact (n < 2^13:
+// Two M-point transforms per row pair or column instead of N^2 products: an image call at N = 1000
+// (5000 points) takes 300 us, 1366 with direct sums; N = 66 to 100 the same either way.  Chirp indices n^2 mod 2N are exact (n < 2^13:
 // no overflow); c is read from the table of W_2N.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ int chirp_index(int n, int N) { return int(unsigned(n) * unsigned(n) % unsigned(2 * N)); }
 
-// B[k] = (transform of conj(c), wrapped)[k] / M, one workgroup; computed in A, stored in T.
-template <typename A, typename T, int LOG2M>
-__global__ __launch_bounds__(FftShape<LOG2M>::NT) void k_chirp_table(int N, const cpx<A>* __restrict__ tw2n,
-                                                                     const cpx<A>* __restrict__ twm, cpx<T>* B) {
+// B[k] = (transform of conj(c), wrapped)[k] / M, one workgroup.
+template <typename T, int LOG2M>
+__global__ __launch_bounds__(FftShape<LOG2M>::NT) void k_chirp_table(int N, const cpx<T>* __restrict__ tw2n,
+                                                                     const cpx<T>* __restrict__ twm, cpx<T>* B) {
     using S = FftShape<LOG2M>;
-    using F = BlockFft<A, LOG2M, false>;
+    using F = BlockFft<T, LOG2M, false>;
     constexpr int M = S::N, NT = S::NT, E = S::E;
-    __shared__ A lds[S::LDS_ELEMS];
+    __shared__ T lds[S::LDS_ELEMS];
     const int tid = threadIdx.x;
-    cpx<A> v[E];
-    F::run(v, lds, tid, M / 2, twm, [&](int n) -> cpx<A> {
+    cpx<T> v[E];
+    F::run(v, lds, tid, M / 2, twm, [&](int n) -> cpx<T> {
         const int m = n < N ? n : M - n;           // |n| of the wrapped sequence
-        return m < N ? cconj(tw2n[chirp_index(m, N)]) : cpx<A>{A(0), A(0)};
+        return m < N ? cconj(tw2n[chirp_index(m, N)]) : cpx<T>{T(0), T(0)};
     });
 #pragma unroll
-    for (int r = 0; r < E; ++r) B[tid + r * NT] = cpx<T>{T(v[r].re / A(M)), T(v[r].im / A(M))};
+    for (int r = 0; r < E; ++r) B[tid + r * NT] = cscale(T(1) / T(M), v[r]);
 }
 
 template <typename T>
@@ -334,8 +334,180 @@ __global__ __launch_bounds__(FftShape<LOG2M>::NT) void k_colpass_chirp(ColArgs<T
 }
 
 // ---------------------------------------------------------------------------
-// even N that neither covers (up to 64, or beyond half the largest workgroup transform and no power of
-// two): direct DFT with exact twiddle indices, O(N) per output.
+// even N, no power of two, in float: direct DFT with exact twiddle indices, each output one chain of fused
+// multiply-adds over n.  (The chirp transform's rounding differs from the chain's by more than the
+// last bits where the result is small: a chain's error follows its largest partial sum.)
+// A thread sums 2 frequencies (256 apart) of 4 rows or columns, so that a twiddle, gathered from the table
+// in LDS, serves 4 sums and its index arithmetic 8 or 16 multiply-adds.  What bounds it: those, and the LDS reads (a
+// gathered table padded against bank conflicts costs more than it saves: 76 + 104 us against 71 + 98).  1000 x 1000
+// pixels: 900 us with one sum per thread and a twiddle from memory for each term, 158 now.
+// ---------------------------------------------------------------------------
+constexpr int DFT_LINES = 4, DFT_FREQS = 512, DFT_STAGE = 256, DFT_AHEAD = 8;
+constexpr int DFT_TILED_MAX = 8192;      // a table of 64 KB: two workgroups per CU
+
+// W_N^(n f) for n = 0, 1, ...: byte offset of the table's entry, (8 n f) mod 8 N
+struct TwiddleWalk {
+    unsigned at, step, end;
+    __device__ __forceinline__ void start(int f, int N, int n) {
+        end = 8u * unsigned(N);
+        step = 8u * unsigned(f);
+        at = 8u * unsigned((long long)n * f % N);
+    }
+    __device__ __forceinline__ cpx<float> next(const unsigned char* tw) {
+        const cpx<float> w = *reinterpret_cast<const cpx<float>*>(tw + at);
+        const unsigned t = at + step;
+        at = min(t, t - end);                      // (t < end: t - end wraps beyond it)
+        return w;
+    }
+};
+
+__device__ __forceinline__ void load_twiddles(unsigned char* lds, const cpx<float>* tw, int N, int tid) {
+    for (int e = tid; e < N; e += 256) reinterpret_cast<cpx<float>*>(lds)[e] = tw[e];
+}
+
+// acc + y w: y real (rows) or complex (columns)
+__device__ __forceinline__ void dft_term(cpx<float>& acc, float y, cpx<float> w) {
+    acc.re = ffma(y, w.re, acc.re);
+    acc.im = ffma(y, w.im, acc.im);
+}
+__device__ __forceinline__ void dft_term(cpx<float>& acc, cpx<float> y, cpx<float> w) {
+    acc.re = ffma(y.re, w.re, ffma(-y.im, w.im, acc.re));
+    acc.im = ffma(y.re, w.im, ffma(y.im, w.re, acc.im));
+}
+
+// Terms from .. to - 1 of a stage (x in LDS) added to the sums; a group of DFT_AHEAD terms is read ahead
+// (1000 x 1000 pixels leave one wave per SIMD: rows and columns 66 + 92 us with 8, 71 + 98 with 4, 95 + 115 with 2).
+template <typename X>
+struct DftTerms {
+    cpx<float> p, q;
+    X y[DFT_LINES];
+};
+template <typename X>
+__device__ __forceinline__ void dft_terms(const X (*x)[DFT_LINES], const unsigned char* tw, TwiddleWalk& wa,
+                                          TwiddleWalk& wb, int from, int to, cpx<float> (&A)[DFT_LINES],
+                                          cpx<float> (&B)[DFT_LINES]) {
+    using Term = DftTerms<X>;
+    const auto read = [&](Term& t, int s) {
+        t.p = wa.next(tw);
+        t.q = wb.next(tw);
+#pragma unroll
+        for (int r = 0; r < DFT_LINES; ++r) t.y[r] = x[s][r];
+    };
+    const auto add = [&](const Term& t) {
+#pragma unroll
+        for (int r = 0; r < DFT_LINES; ++r) {
+            dft_term(A[r], t.y[r], t.p);
+            dft_term(B[r], t.y[r], t.q);
+        }
+    };
+    constexpr int G = DFT_AHEAD;
+    int s = from;
+    if (to - from >= G) {
+        Term cur[G];
+#pragma unroll
+        for (int g = 0; g < G; ++g) read(cur[g], s + g);
+#pragma unroll 2
+        for (; s + 2 * G <= to; s += G) {
+            Term nxt[G];
+#pragma unroll
+            for (int g = 0; g < G; ++g) read(nxt[g], s + G + g);
+#pragma unroll
+            for (int g = 0; g < G; ++g) add(cur[g]);
+#pragma unroll
+            for (int g = 0; g < G; ++g) cur[g] = nxt[g];
+        }
+#pragma unroll
+        for (int g = 0; g < G; ++g) add(cur[g]);
+        s += G;
+    }
+    for (; s < to; ++s) {
+        Term t;
+        read(t, s);
+        add(t);
+    }
+}
+
+// All 2 Rs terms of DFT_LINES lines at frequencies fa and fb; load(s, x) fills a term's values.
+template <typename X, typename Load>
+__device__ __forceinline__ void dft_tile(X (*x)[DFT_LINES], const unsigned char* tw, int N, int Rs, int fa, int fb,
+                                         cpx<float> (&A)[DFT_LINES], cpx<float> (&B)[DFT_LINES], Load&& load) {
+    const int tid = threadIdx.x;
+    TwiddleWalk wa, wb;
+    wa.start(fa, N, 0);
+    wb.start(fb, N, 0);
+    X y[DFT_LINES];
+    if (tid < 2 * Rs) load(tid, y);
+    for (int s0 = 0; s0 < 2 * Rs; s0 += DFT_STAGE) {
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < DFT_LINES; ++r) x[tid][r] = y[r];
+        __syncthreads();
+        if (s0 + DFT_STAGE + tid < 2 * Rs) load(s0 + DFT_STAGE + tid, y);
+        const int end = min(DFT_STAGE, 2 * Rs - s0), cut = min(max(Rs - s0, 0), end);
+        dft_terms(x, tw, wa, wb, 0, cut, A, B);
+        if (s0 <= Rs && Rs < s0 + end) {           // (the support goes on at n = N - Rs)
+            wa.start(fa, N, N - Rs);
+            wb.start(fb, N, N - Rs);
+        }
+        dft_terms(x, tw, wa, wb, cut, end, A, B);
+    }
+}
+
+template <int SRC>
+__global__ __launch_bounds__(256) void k_rowdft_tiled(RowArgs<float> a) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];    // twiddle table
+    __shared__ __align__(16) float x[DFT_STAGE][DFT_LINES];
+    const int N = a.N, Rs = a.Rs, C = N / 2 + 1, tid = threadIdx.x;
+    const int kk0 = DFT_LINES * blockIdx.x, l0 = DFT_FREQS * blockIdx.y + tid;
+    load_twiddles(smem_raw, a.tw, N, tid);
+    int k[DFT_LINES];
+#pragma unroll
+    for (int r = 0; r < DFT_LINES; ++r) k[r] = compact_to_row(min(kk0 + r, 2 * Rs - 1), Rs, N);
+    cpx<float> A[DFT_LINES] = {}, B[DFT_LINES] = {};
+    dft_tile(x, smem_raw, N, Rs, min(l0, C - 1), min(l0 + 256, C - 1), A, B, [&](int s, float (&y)[DFT_LINES]) {
+        const int n = s < Rs ? s : s + N - 2 * Rs;
+#pragma unroll
+        for (int r = 0; r < DFT_LINES; ++r) y[r] = row_source<float, SRC>(a, k[r], n);
+    });
+#pragma unroll
+    for (int r = 0; r < DFT_LINES; ++r) {
+        if (kk0 + r >= 2 * Rs) break;
+        cpx<float>* out = a.Tm + size_t(kk0 + r) * a.ldT;
+        if (l0 < C) out[l0] = A[r];
+        if (l0 + 256 < C) out[l0 + 256] = B[r];
+    }
+}
+
+// (the row spectra are padded to whole groups of four columns)
+template <int OUT>
+__global__ __launch_bounds__(256) void k_coldft_tiled(ColArgs<float> a) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];    // twiddle table
+    __shared__ __align__(16) cpx<float> x[DFT_STAGE][DFT_LINES];
+    const int N = a.N, Rs = a.Rs, C = N / 2 + 1, tid = threadIdx.x;
+    const int c0 = DFT_LINES * blockIdx.x, k0 = DFT_FREQS * blockIdx.y + tid;
+    load_twiddles(smem_raw, a.tw, N, tid);
+    cpx<float> A[DFT_LINES] = {}, B[DFT_LINES] = {};
+    dft_tile(x, smem_raw, N, Rs, min(k0, N - 1), min(k0 + 256, N - 1), A, B, [&](int s, cpx<float> (&y)[DFT_LINES]) {
+        const cpx<float>* src = a.Tm + size_t(s) * a.ldT + c0;
+#pragma unroll
+        for (int c = 0; c < DFT_LINES; ++c) y[c] = src[c];
+    });
+    const auto store = [&](int col, int k, cpx<float> X) {
+        if (col >= C || k >= N) return;
+        if constexpr (OUT == OUT_COLMAJOR_SHIFT) a.S[size_t(col) * a.ldS + (k < N / 2 ? k + N / 2 : k - N / 2)] = X;
+        else a.S[size_t(k) * C + col] = X;
+    };
+#pragma unroll
+    for (int c = 0; c < DFT_LINES; ++c) {
+        store(c0 + c, k0, A[c]);
+        store(c0 + c, k0 + 256, B[c]);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// even N that none of these covers (in double up to 64, or beyond half the largest workgroup transform and no
+// power of two; in float no power of two whose twiddle table LDS does not hold beside the others'): as
+// above, one output at a time.
 // ---------------------------------------------------------------------------
 template <typename T, int SRC>
 __global__ __launch_bounds__(256) void k_rowdft_generic(RowArgs<T> a) {
