@@ -1837,7 +1837,7 @@ void batch_tune(BatchPlan<T>& P, hipStream_t s, int W, int mode, typename BatchP
             best.chunk = c;
         }
         // chunks too small to fill the chip only get slower with every halving (up to twice the best time
-        // and more): 256 walkers x 3 datasets spend 176 ms in this search with them, 80 without
+        // and more): the first call for 256 walkers x 3 datasets takes 176 ms with them, 78 without
         if (ms > 1.25f * tbest) break;
     }
     auto try_shape = [&](BatchShape t) {

@@ -53,7 +53,7 @@ __device__ __forceinline__ void atomic_add_f64(double* p, double v) { unsafeAtom
 // tile (by workgroup index), which the adjoint column pass folds into Hh.
 //
 // What bounds it: those requests and, where the points are dense, vector instruction issue (about
-// 330 instructions per 64 points).  A thread takes GPT points: the bounding box, the
+// 260 instructions per 64 points with GPT 2, 417 with 1; 650 before).  A thread takes GPT points: the bounding box, the
 // window's clearing and flush and the wave reductions are paid once per GPT points.
 // ---------------------------------------------------------------------------
 constexpr int GHOT = 16;          // hot tile: columns [0, GHOT) x folded rows [0, GHOT)

@@ -220,8 +220,8 @@ __global__ __launch_bounds__(FftShape<LOG2N>::NT) void k_colpass(ColArgs<T> a) {
 // a convolution that a cyclic one of M >= 2N - 1 points holds: transform of x c (M points, a power of two,
 // BlockFft), times the transform B of conj(c) (k_chirp_table, scaled by 1/M), transform back, times c.
 // Two M-point transforms per row pair or column instead of N^2 products: an image call at N = 1000
-// (5000 points) takes 300 us, 1366 with direct sums; N = 66 to 100 the same either way.  Chirp indices n^2 mod 2N are exact (n < 2^13:
-// no overflow); c is read from the table of W_2N.
+// (5000 points) takes 300 us, 1366 with direct sums; N = 66 to 100 the same either way.  Chirp indices
+// n^2 mod 2N are exact (n < 2^13: no overflow); c is read from the table of W_2N.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ int chirp_index(int n, int N) { return int(unsigned(n) * unsigned(n) % unsigned(2 * N)); }
 
