@@ -216,7 +216,8 @@ __device__ __forceinline__ void sample_grad_sym_body(const SampleArgs<T>& a, con
     const int wp = pmax - pmin + 1, w2 = 2 * (mmax - mmin + 1);
     const bool use_win = any && wp * w2 <= WIN;      // (wp, w2 <= 2^14, no overflow)
     const int nwin = use_win ? wp * w2 : 0;          // even
-    for (int j = 2 * tid; j < (use_win ? nwin : WIN); j += 512)
+    const int nclear = use_win ? nwin : GPT == 1 && g.direct ? GHOT * GHOT : WIN;
+    for (int j = 2 * tid; j < nclear; j += 512)
         *reinterpret_cast<cpx<double>*>(&win[j]) = cpx<double>{0.0, 0.0};
     double* rep = g.hot + size_t(blk % GREP) * (GHOT * GHOT);
     __syncthreads();
@@ -266,6 +267,28 @@ __device__ __forceinline__ void sample_grad_sym_body(const SampleArgs<T>& a, con
                 lds_add_f64(&win[o2 + dm], x3);
             }
         }
+    } else if (GPT == 1 && g.direct) {
+        // Sparse points of a small call: straight to Hh, a point's four corners by a lane quad (they lie in one
+        // 32-byte run when the lower column is even, h_index): in round r, lane l carries corner l & 3 of point
+        // (l >> 2) + 16 r of its wave.  Cells of the hot tile are summed in LDS first.
+        const int corner = lane & 3;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int src = (lane >> 2) + 16 * r;
+            const int iu = __shfl(pt[0].iu, src, 64), d = __shfl(pt[0].d, src, 64);
+            const double x0 = __shfl(pt[0].g[0], src, 64), x1 = __shfl(pt[0].g[1], src, 64);
+            const double x2 = __shfl(pt[0].g[2], src, 64), x3 = __shfl(pt[0].g[3], src, 64);
+            const double xl = corner & 1 ? x1 : x0, xh = corner & 1 ? x3 : x2;
+            const double x = corner & 2 ? xh : xl;
+            const int col = iu + (corner >> 1), m = corner & 1 ? row_hi(d) : row_lo(d);
+            if (iu >= 0 && x != 0.0) {
+                if (col < GHOT && m < GHOT) lds_add_f64(&win[col * GHOT + m], x);
+                else atomic_add_f64(g.Hh + h_index(col, m, a.ldH), x);
+            }
+        }
+        __syncthreads();
+        static_assert(GHOT * GHOT == 256, "one cell per thread");
+        if (win[tid] != 0.0) atomic_add_f64(rep + tid, win[tid]);
     } else {
         // Sparse points: a table of 64-byte lines of Hh (2 columns x 4 rows, h_index), open addressing,
         // built and flushed for one block of 256 points at a time.
@@ -276,22 +299,6 @@ __device__ __forceinline__ void sample_grad_sym_body(const SampleArgs<T>& a, con
                 if (j == k) p = pt[j];
             for (int j = tid; j < NLINE; j += 256) keys[j] = EMPTY;
             __syncthreads();
-            if (g.direct) {
-                if (p.iu >= 0) {
-                    const int m0 = row_lo(p.d), m1 = row_hi(p.d);
-                    const auto add = [&](int col, int m, double x) {
-                        if (x == 0.0) return;
-                        double* to = g.Hh + h_index(col, m, a.ldH);
-                        if (col < GHOT && m < GHOT) to = rep + col * GHOT + m;
-                        atomic_add_f64(to, x);
-                    };
-                    add(p.iu, m0, p.g[0]);
-                    add(p.iu, m1, p.g[1]);
-                    add(p.iu + 1, m0, p.g[2]);
-                    add(p.iu + 1, m1, p.g[3]);
-                }
-                continue;
-            }
             if (p.iu >= 0) {
                 const int m0 = row_lo(p.d), m1 = row_hi(p.d);
                 const unsigned ld4 = unsigned(a.ldH) >> 2;
@@ -405,10 +412,11 @@ __device__ __forceinline__ void sample_grad_sym_body(const SampleArgs<T>& a, con
 constexpr int GPT_SINGLE = 1, GPT_BATCH = 2;
 // Batched launches of at most this many one-point workgroups take one point per thread too.
 constexpr size_t GRAD_FEW_WORKGROUPS = 8192;
-// One call with at most this many blocks of points adds its sparse points straight to Hh: the line table
-// costs such a call, which is one workgroup's latency, 1.9 us (5003 points at nxy = 512: 6.9 against
-// 5.0 us), the atomics of 8192 sparse points at four requests each about as much.
-constexpr int GRAD_DIRECT_BLOCKS = 32;
+// Launches of at most this many workgroups add their sparse points straight to Hh: all of them are resident at once, so
+// the launch takes one workgroup's latency, to which the line table's building and flush add 2 to 4 us, while the
+// atomics' rate does not bind yet.  nxy = 4096, direct against table: 8000 points 4.9 / 8.4 us, 64000 7.1 / 8.4,
+// 128000 11.1 / 10.2, 256000 14.4 / 13.0; nxy = 1024: 8000 4.4 / 9.4, 128000 6.2 / 9.4.
+constexpr int GRAD_DIRECT_BLOCKS = 512;
 template <typename T>
 __global__ __launch_bounds__(256) void k_sample_grad_sym(SampleArgs<T> a, GradArgs<T> g) {
     sample_grad_sym_body<T, T, GWIN, GPT_SINGLE>(a, a, g, blockIdx.x);

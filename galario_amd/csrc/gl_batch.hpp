@@ -252,7 +252,8 @@ __global__ __launch_bounds__(256) void k_sample_grad_sym_b(SampleArgs<T> a, Batc
     const int slot = blockIdx.y, w = b.w0 + slot;
     walker_sample_args(a, b, slot, w);
     double* hh = b.Hh + slot * b.sHh;
-    const GradArgs<T> g{hh, hh + b.hot_off, b.part + size_t(w) * 4 * b.ldPart + b.partOff, b.ldPart, nblocks, 0};
+    const GradArgs<T> g{hh, hh + b.hot_off, b.part + size_t(w) * 4 * b.ldPart + b.partOff, b.ldPart, nblocks,
+                        GPT == 1 && nblocks * int(gridDim.y) <= GRAD_DIRECT_BLOCKS};
     if constexpr (MIX) sample_grad_sym_body<T, double, WIN, GPT>(a, walker_scalars_f64(a, b, w), g, blockIdx.x);
     else sample_grad_sym_body<T, T, WIN, GPT>(a, a, g, blockIdx.x);
 }

@@ -73,10 +73,11 @@ def test_gradient_beside_invalid_point():
     assert ta.take_oob_flag()
 
 
-# up to 32 blocks of 256 points the sparse ones go straight to memory, beyond through the line table; in locality
+# up to 512 blocks of 256 points the sparse ones go straight to memory, beyond through the line table; in locality
 # order the dense ones take the window, in random order no workgroup's cells fit it and the table overflows
 @pytest.mark.parametrize('sort', [True, False])
-@pytest.mark.parametrize('N, n', [(256, 1), (256, 257), (256, 8192), (256, 8193), (1024, 8192), (1024, 20011)])
+@pytest.mark.parametrize('N, n', [(256, 1), (256, 257), (256, 8193), (1024, 20011), (256, 131072), (256, 131073),
+                                  (1024, 131072), (1024, 131073)])
 def test_gradient_scatter(N, n, sort):
     I, dR = profile()
     p = points(n, N, 1.0, 0.45 * N)
@@ -87,8 +88,8 @@ def test_gradient_scatter(N, n, sort):
     assert got[0].item() == ds.chi2_profile(It, RMIN, dR, N, DXY, **kw()).item()      # (one order of sums)
 
 
-# one and two points per thread (up to 8192 workgroups of one block each, and more), each LDS window
-@pytest.mark.parametrize('walkers, n', [(2, 20011), (110, 20011)])
+# straight to memory (up to 512 workgroups), one and two points per thread (up to 8192 and more), each LDS window
+@pytest.mark.parametrize('walkers, n', [(2, 20011), (7, 20011), (110, 20011)])
 @pytest.mark.parametrize('window', [2048, 3072, 4096])
 def test_batched_gradient_scatter(walkers, n, window):
     from galario_amd import torch_api as ta
