@@ -165,9 +165,6 @@ struct Workspace {
     DevBuf Tm, S, part, flag_dev, pack;
     DevBuf Hh, Th;                // gradient: adjoint half spectrum (kept zero between calls), adjoint rows
     bool Hh_zero = false;         // Hh holds zeros (cleared by the adjoint column pass)
-    DevBuf chirp;                 // transform of the last chirp used (k_chirp_table) ...
-    int chirp_n = 0;              // ... for this N (0: none)
-    bool chirp_captured = false;  // a captured graph writes it too: rebuilt by every call
     DevBuf in[8];
     DevBuf out;
     double* h_scal = nullptr;     // pinned: [0] result, [1] flag; the host-array calls' kernels write them there
@@ -177,9 +174,6 @@ struct Workspace {
     void release() {
         Tm.release(); S.release(); part.release(); pack.release(); Hh.release(); Th.release();
         Hh_zero = false;
-        chirp.release();
-        chirp_n = 0;
-        chirp_captured = false;
         flag_dev.release(); out.release();
         for (auto& b : in) b.release();
         if (h_scal) (void)hipHostFree(h_scal);
@@ -454,52 +448,6 @@ void launch_colpass(int L, int blocks, hipStream_t s, const ColArgs<T>& a) {
     }
 }
 
-// log2 of the power of two M >= 2N - 1 of the chirp transform, -1 where the direct sums serve: float, N up to 64
-// (which they do in less time than the chirp transform's longer path) or M beyond the largest transform.
-template <typename T>
-int chirp_log2(int N) {
-    if (sizeof(T) == 4 || N <= 64) return -1;
-    int L = 7;
-    while (L <= max_fast_log2<T>() && (1 << L) < 2 * N - 1) ++L;
-    return L <= max_fast_log2<T>() ? L : -1;
-}
-
-// Tables of the chirp transform of size N = a.N.  B is kept in the thread's workspace, whose calls run in order,
-// and rebuilt when N changes.
-ChirpArgs<double> chirp_tables(Workspace& w, hipStream_t s, int N, int L) {
-    cpx<double>* B = w.chirp.get<cpx<double>>(size_t(1) << L);
-    if (s) {
-        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-        HC(hipStreamIsCapturing(s, &st));
-        if (st != hipStreamCaptureStatusNone) w.chirp_captured = true;
-    }
-    const cpx<double>*tw2n = twiddles<double>(2 * N), *twm = twiddles<double>(1 << L);
-    if (w.chirp_captured || w.chirp_n != N) {
-        w.chirp_n = 0;
-#define GL_CALL(LL) \
-    hipLaunchKernelGGL((k_chirp_table<double, LL>), dim3(1), dim3(FftShape<LL>::NT), 0, s, N, tw2n, twm, B)
-        GL_L_SWITCH(double, GL_CALL)
-#undef GL_CALL
-        HC(hipGetLastError());
-        w.chirp_n = N;
-    }
-    return ChirpArgs<double>{tw2n, twm, B};
-}
-
-template <int SRC>
-void launch_rowpass_chirp(int L, int pairs, hipStream_t s, const RowArgs<double>& a, const ChirpArgs<double>& c) {
-#define GL_CALL(LL) hipLaunchKernelGGL((k_rowpass_chirp<double, LL, SRC>), dim3(pairs), dim3(FftShape<LL>::NT), 0, s, a, c)
-    GL_L_SWITCH(double, GL_CALL)
-#undef GL_CALL
-}
-
-template <int OUT>
-void launch_colpass_chirp(int L, int blocks, hipStream_t s, const ColArgs<double>& a, const ChirpArgs<double>& c) {
-#define GL_CALL(LL) hipLaunchKernelGGL((k_colpass_chirp<double, LL, OUT>), dim3(blocks), dim3(FftShape<LL>::NT), 0, s, a, c)
-    GL_L_SWITCH(double, GL_CALL)
-#undef GL_CALL
-}
-
 inline unsigned blocks_for(size_t n, unsigned per) { return unsigned((n + per - 1) / per); }
 
 template <typename K>
@@ -521,33 +469,24 @@ cpx<T>* build_spectrum(Workspace& w, hipStream_t s, RowArgs<T> ra, int N, int Rs
     ra.ldT = ldT;
     ra.Tm = Tm;
     ColArgs<T> ca{Tm, N, Rs, ldT, nullptr, S_out, ldS};
-    const int L = fast_log2<T>(N), LM = L > 0 ? -1 : chirp_log2<T>(N);
-    if (LM < 0) ra.tw = ca.tw = twiddles<T>(N);
-    if (LM > 0) {
-        if constexpr (sizeof(T) == 8) {
-            const ChirpArgs<T> c = chirp_tables(w, s, N, LM);
-            t_timer.mark(ST_ROW, s);
-            launch_rowpass_chirp<SRC>(LM, Rs, s, ra, c);
-            t_timer.mark(ST_COL, s);
-            launch_colpass_chirp<OUT>(LM, 8 * ((C + 7) / 8), s, ca, c);
-        }
-    } else if (L > 0) {
+    const int L = fast_log2<T>(N);
+    ra.tw = ca.tw = twiddles<T>(N);
+    const size_t table = sizeof(cpx<T>) * size_t(N);
+    if (L > 0) {
         t_timer.mark(ST_ROW, s);
         launch_rowpass<T, SRC>(L, Rs, s, ra);
         t_timer.mark(ST_COL, s);
         launch_colpass<T, OUT>(L, 8 * ((C + 7) / 8), s, ca);
-    } else if (sizeof(T) == 4 && N <= DFT_TILED_MAX) {
-        if constexpr (sizeof(T) == 4) {
-            const size_t lds = sizeof(cpx<T>) * size_t(N);
-            allow_lds(k_rowdft_tiled<SRC>, lds);
-            allow_lds(k_coldft_tiled<OUT>, lds);
-            t_timer.mark(ST_ROW, s);
-            hipLaunchKernelGGL((k_rowdft_tiled<SRC>), dim3((2 * Rs + DFT_LINES - 1) / DFT_LINES, (C + DFT_FREQS - 1) / DFT_FREQS),
-                               dim3(256), lds, s, ra);
-            t_timer.mark(ST_COL, s);
-            hipLaunchKernelGGL((k_coldft_tiled<OUT>), dim3((C + DFT_LINES - 1) / DFT_LINES, (N + DFT_FREQS - 1) / DFT_FREQS),
-                               dim3(256), lds, s, ca);
-        }
+    } else if (table <= DFT_TABLE_BYTES) {
+        allow_lds(k_rowdft_tiled<T, SRC>, table);
+        allow_lds(k_coldft_tiled<T, OUT>, table);
+        t_timer.mark(ST_ROW, s);
+        hipLaunchKernelGGL((k_rowdft_tiled<T, SRC>),
+                           dim3((2 * Rs + DFT_LINES - 1) / DFT_LINES, (C + DFT_FREQS - 1) / DFT_FREQS), dim3(256), table, s,
+                           ra);
+        t_timer.mark(ST_COL, s);
+        hipLaunchKernelGGL((k_coldft_tiled<T, OUT>),
+                           dim3((C + DFT_LINES - 1) / DFT_LINES, (N + DFT_FREQS - 1) / DFT_FREQS), dim3(256), table, s, ca);
     } else {
         const size_t lds_row = sizeof(T) * size_t(2 * Rs);
         if (lds_row > 160 * 1024) fail(GALARIO_ERR_INVALID, "Error in fft: image size not supported");

@@ -353,13 +353,6 @@ struct BlockFft {
         if constexpr (LOADS_LDS) __syncthreads();
         rest<1>(v, lds, tid, tw, only0);
     }
-
-    // The same of inputs already in registers: v[r] = element tid + r*N/E.
-    static __device__ __forceinline__ void run_registers(cpx<T> (&v)[E], T* lds, int tid,
-                                                         const cpx<T>* __restrict__ tw) {
-        dft<E, INV>(v);
-        rest<1>(v, lds, tid, tw, false);
-    }
 };
 
 // One wave's 512-point transform at the fractional frequencies K + k0/P

@@ -215,178 +215,70 @@ __global__ __launch_bounds__(FftShape<LOG2N>::NT) void k_colpass(ColArgs<T> a) {
 }
 
 // ---------------------------------------------------------------------------
-// other even N in double: Bluestein's chirp transform.  With c[n] = exp(-i pi n^2 / N),
-//   X[k] = c[k] sum_n (x[n] c[n]) conj(c[k - n]),
-// a convolution that a cyclic one of M >= 2N - 1 points holds: transform of x c (M points, a power of two,
-// BlockFft), times the transform B of conj(c) (k_chirp_table, scaled by 1/M), transform back, times c.
-// Two M-point transforms per row pair or column instead of N^2 products: an image call at N = 1000
-// (5000 points) takes 300 us, 1366 with direct sums; N = 66 to 100 the same either way.  Chirp indices
-// n^2 mod 2N are exact (n < 2^13: no overflow); c is read from the table of W_2N.
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ int chirp_index(int n, int N) { return int(unsigned(n) * unsigned(n) % unsigned(2 * N)); }
-
-// B[k] = (transform of conj(c), wrapped)[k] / M, one workgroup.
-template <typename T, int LOG2M>
-__global__ __launch_bounds__(FftShape<LOG2M>::NT) void k_chirp_table(int N, const cpx<T>* __restrict__ tw2n,
-                                                                     const cpx<T>* __restrict__ twm, cpx<T>* B) {
-    using S = FftShape<LOG2M>;
-    using F = BlockFft<T, LOG2M, false>;
-    constexpr int M = S::N, NT = S::NT, E = S::E;
-    __shared__ T lds[S::LDS_ELEMS];
-    const int tid = threadIdx.x;
-    cpx<T> v[E];
-    F::run(v, lds, tid, M / 2, twm, [&](int n) -> cpx<T> {
-        const int m = n < N ? n : M - n;           // |n| of the wrapped sequence
-        return m < N ? cconj(tw2n[chirp_index(m, N)]) : cpx<T>{T(0), T(0)};
-    });
-#pragma unroll
-    for (int r = 0; r < E; ++r) B[tid + r * NT] = cscale(T(1) / T(M), v[r]);
-}
-
-template <typename T>
-struct ChirpArgs {
-    const cpx<T>* tw2n;      // W_2N^e
-    const cpx<T>* twm;       // W_M^e
-    const cpx<T>* B;         // k_chirp_table
-};
-
-// The N-point transform of x[n] = load(n) (0 <= n < N) by one workgroup: on return v[r] holds X[tid + r M/E]
-// where that index is below N; every thread has finished reading LDS.
-template <typename T, int LOG2M, typename Loader>
-__device__ __forceinline__ void chirp_transform(cpx<T> (&v)[FftShape<LOG2M>::E], T* lds, int tid, int N,
-                                                const ChirpArgs<T>& c, Loader&& load) {
-    using S = FftShape<LOG2M>;
-    BlockFft<T, LOG2M, false>::run(v, lds, tid, S::N / 2, c.twm, [&](int n) -> cpx<T> {
-        return n < N ? cmul(load(n), c.tw2n[chirp_index(n, N)]) : cpx<T>{T(0), T(0)};
-    });
-#pragma unroll
-    for (int r = 0; r < S::E; ++r) v[r] = cmul(v[r], c.B[tid + r * S::NT]);
-    BlockFft<T, LOG2M, true>::run_registers(v, lds, tid, c.twm);
-#pragma unroll
-    for (int r = 0; r < S::E; ++r) {
-        const int k = tid + r * S::NT;
-        if (k < N) v[r] = cmul(v[r], c.tw2n[chirp_index(k, N)]);
-    }
-}
-
-// Two real rows as one complex transform (as k_rowpass).
-template <typename T, int LOG2M, int SRC>
-__global__ __launch_bounds__(FftShape<LOG2M>::NT) void k_rowpass_chirp(RowArgs<T> a, ChirpArgs<T> c) {
-    using S = FftShape<LOG2M>;
-    constexpr int NT = S::NT, E = S::E;
-    __shared__ T lds[S::LDS_ELEMS];
-    const int tid = threadIdx.x, N = a.N, Rs = a.Rs;
-    const int kk_a = 2 * blockIdx.x, kk_b = kk_a + 1;
-    const int ka = compact_to_row(kk_a, Rs, N), kb = compact_to_row(kk_b, Rs, N);
-    cpx<T> v[E];
-    chirp_transform<T, LOG2M>(v, lds, tid, N, c, [&](int n) -> cpx<T> {
-        if (n >= Rs && n < N - Rs) return cpx<T>{T(0), T(0)};
-        return cpx<T>{row_source<T, SRC>(a, ka, n), row_source<T, SRC>(a, kb, n)};
-    });
-    // X_a[l] = (Z[l] + conj Z[N-l]) / 2, X_b[l] = (Z[l] - conj Z[N-l]) / 2i, one component at a time
-    const int C = N / 2 + 1;
-    cpx<T>* outa = a.Tm + size_t(kk_a) * a.ldT;
-    cpx<T>* outb = a.Tm + size_t(kk_b) * a.ldT;
-#pragma unroll
-    for (int r = 0; r < E; ++r)
-        if (tid + r * NT < N) lds[lpad(tid + r * NT)] = v[r].re;
-    __syncthreads();
-    for (int l = tid; l < C; l += NT) {
-        const T zr = lds[lpad(l)], wr = lds[lpad(l ? N - l : 0)];
-        outa[l].re = T(0.5) * (zr + wr);
-        outb[l].im = T(0.5) * (wr - zr);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < E; ++r)
-        if (tid + r * NT < N) lds[lpad(tid + r * NT)] = v[r].im;
-    __syncthreads();
-    for (int l = tid; l < C; l += NT) {
-        const T zi = lds[lpad(l)], wi = lds[lpad(l ? N - l : 0)];
-        outa[l].im = T(0.5) * (zi - wi);
-        outb[l].re = T(0.5) * (zi + wi);
-    }
-}
-
-template <typename T, int LOG2M, int OUT>
-__global__ __launch_bounds__(FftShape<LOG2M>::NT) void k_colpass_chirp(ColArgs<T> a, ChirpArgs<T> c) {
-    using S = FftShape<LOG2M>;
-    constexpr int NT = S::NT, E = S::E;
-    __shared__ T lds[S::LDS_ELEMS];
-    const int tid = threadIdx.x, N = a.N, Rs = a.Rs, C = N / 2 + 1;
-    const int col = xcd_column(blockIdx.x, gridDim.x);
-    if (col >= C) return;
-    const cpx<T>* src = a.Tm + col;
-    const size_t ldT = a.ldT;
-    cpx<T> v[E];
-    chirp_transform<T, LOG2M>(v, lds, tid, N, c, [&](int n) -> cpx<T> {
-        if (n >= Rs && n < N - Rs) return cpx<T>{T(0), T(0)};
-        return src[size_t(n < Rs ? n : n - N + 2 * Rs) * ldT];
-    });
-#pragma unroll
-    for (int r = 0; r < E; ++r) {
-        const int k = tid + r * NT;
-        if (k < N) {
-            if constexpr (OUT == OUT_COLMAJOR_SHIFT) a.S[size_t(col) * a.ldS + (k < N / 2 ? k + N / 2 : k - N / 2)] = v[r];
-            else a.S[size_t(k) * C + col] = v[r];
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------
-// even N, no power of two, in float: direct DFT with exact twiddle indices, each output one chain of fused
-// multiply-adds over n.  (The chirp transform's rounding differs from the chain's by more than the
-// last bits where the result is small: a chain's error follows its largest partial sum.)
+// other even N: direct DFT with exact twiddle indices, each output one chain of fused multiply-adds over n.
+// (A fast transform of such a size, Bluestein's with two power-of-two transforms, errs 4 to 6 times as much in the weak
+// cells, the long baselines: its errors follow the strongest cell, a chain's its own largest partial sum. 400 x 400
+// pixels of a compact source in double, median error of the cells below 1e-3 of the peak: 4.3e-15 against 6.7e-16.)
 // A thread sums 2 frequencies (256 apart) of 4 rows or columns, so that a twiddle, gathered from the table
 // in LDS, serves 4 sums and its index arithmetic 8 or 16 multiply-adds.  What bounds it: those, and the LDS reads (a
-// gathered table padded against bank conflicts costs more than it saves: 76 + 104 us against 71 + 98).  1000 x 1000
-// pixels: 900 us with one sum per thread and a twiddle from memory for each term, 158 now.
+// gathered table padded against bank conflicts costs more than it saves: in float 76 + 104 us against 71 + 98).
+// 1000 x 1000 pixels: with one sum per thread and a twiddle from memory for each term 900 us in float and a sampleImage call of
+// 1400 us in double; 158 us (double: 86 + 126) and a call of 480 us now.
 // ---------------------------------------------------------------------------
-constexpr int DFT_LINES = 4, DFT_FREQS = 512, DFT_STAGE = 256, DFT_AHEAD = 8;
-constexpr int DFT_TILED_MAX = 8192;      // a table of 64 KB: two workgroups per CU
+constexpr int DFT_LINES = 4, DFT_FREQS = 512, DFT_STAGE = 256;
+constexpr size_t DFT_TABLE_BYTES = 65536;   // largest table: two workgroups per CU
 
-// W_N^(n f) for n = 0, 1, ...: byte offset of the table's entry, (8 n f) mod 8 N
+// W_N^(n f) for n = 0, 1, ...: byte offset of the table's entry, B n f mod B N for entries of B bytes
+template <typename T>
 struct TwiddleWalk {
+    static constexpr unsigned B = sizeof(cpx<T>);
     unsigned at, step, end;
     __device__ __forceinline__ void start(int f, int N, int n) {
-        end = 8u * unsigned(N);
-        step = 8u * unsigned(f);
-        at = 8u * unsigned((long long)n * f % N);
+        end = B * unsigned(N);
+        step = B * unsigned(f);
+        at = B * unsigned((long long)n * f % N);
     }
-    __device__ __forceinline__ cpx<float> next(const unsigned char* tw) {
-        const cpx<float> w = *reinterpret_cast<const cpx<float>*>(tw + at);
+    __device__ __forceinline__ cpx<T> next(const unsigned char* tw) {
+        const cpx<T> w = *reinterpret_cast<const cpx<T>*>(tw + at);
         const unsigned t = at + step;
         at = min(t, t - end);                      // (t < end: t - end wraps beyond it)
         return w;
     }
 };
 
-__device__ __forceinline__ void load_twiddles(unsigned char* lds, const cpx<float>* tw, int N, int tid) {
-    for (int e = tid; e < N; e += 256) reinterpret_cast<cpx<float>*>(lds)[e] = tw[e];
+template <typename T>
+__device__ __forceinline__ void load_twiddles(unsigned char* lds, const cpx<T>* tw, int N, int tid) {
+    for (int e = tid; e < N; e += 256) reinterpret_cast<cpx<T>*>(lds)[e] = tw[e];
 }
 
 // acc + y w: y real (rows) or complex (columns)
-__device__ __forceinline__ void dft_term(cpx<float>& acc, float y, cpx<float> w) {
+template <typename T>
+__device__ __forceinline__ void dft_term(cpx<T>& acc, T y, cpx<T> w) {
     acc.re = ffma(y, w.re, acc.re);
     acc.im = ffma(y, w.im, acc.im);
 }
-__device__ __forceinline__ void dft_term(cpx<float>& acc, cpx<float> y, cpx<float> w) {
+template <typename T>
+__device__ __forceinline__ void dft_term(cpx<T>& acc, cpx<T> y, cpx<T> w) {
     acc.re = ffma(y.re, w.re, ffma(-y.im, w.im, acc.re));
     acc.im = ffma(y.re, w.im, ffma(y.im, w.re, acc.im));
 }
 
-// Terms from .. to - 1 of a stage (x in LDS) added to the sums; a group of DFT_AHEAD terms is read ahead
-// (1000 x 1000 pixels leave one wave per SIMD: rows and columns 66 + 92 us with 8, 71 + 98 with 4, 95 + 115 with 2).
-template <typename X>
+// Terms from .. to - 1 of a stage (x in LDS) added to the sums; a group of dft_ahead terms is read ahead
+// (1000 x 1000 pixels leave one wave per SIMD: in float rows and columns 66 + 92 us with 8, 71 + 98 with 4, 95 + 115 with
+// 2; in double a sampleImage call takes 481 us with 4, 490 with 2, and at 2000 x 2000, 2.46 and 2.27 ms).
+template <typename T>
+constexpr int dft_ahead() { return sizeof(T) == 4 ? 8 : 4; }
+
+template <typename T, typename X>
 struct DftTerms {
-    cpx<float> p, q;
+    cpx<T> p, q;
     X y[DFT_LINES];
 };
-template <typename X>
-__device__ __forceinline__ void dft_terms(const X (*x)[DFT_LINES], const unsigned char* tw, TwiddleWalk& wa,
-                                          TwiddleWalk& wb, int from, int to, cpx<float> (&A)[DFT_LINES],
-                                          cpx<float> (&B)[DFT_LINES]) {
-    using Term = DftTerms<X>;
+template <typename T, typename X>
+__device__ __forceinline__ void dft_terms(const X (*x)[DFT_LINES], const unsigned char* tw, TwiddleWalk<T>& wa,
+                                          TwiddleWalk<T>& wb, int from, int to, cpx<T> (&A)[DFT_LINES],
+                                          cpx<T> (&B)[DFT_LINES]) {
+    using Term = DftTerms<T, X>;
     const auto read = [&](Term& t, int s) {
         t.p = wa.next(tw);
         t.q = wb.next(tw);
@@ -400,7 +292,7 @@ __device__ __forceinline__ void dft_terms(const X (*x)[DFT_LINES], const unsigne
             dft_term(B[r], t.y[r], t.q);
         }
     };
-    constexpr int G = DFT_AHEAD;
+    constexpr int G = dft_ahead<T>();
     int s = from;
     if (to - from >= G) {
         Term cur[G];
@@ -428,11 +320,11 @@ __device__ __forceinline__ void dft_terms(const X (*x)[DFT_LINES], const unsigne
 }
 
 // All 2 Rs terms of DFT_LINES lines at frequencies fa and fb; load(s, x) fills a term's values.
-template <typename X, typename Load>
+template <typename T, typename X, typename Load>
 __device__ __forceinline__ void dft_tile(X (*x)[DFT_LINES], const unsigned char* tw, int N, int Rs, int fa, int fb,
-                                         cpx<float> (&A)[DFT_LINES], cpx<float> (&B)[DFT_LINES], Load&& load) {
+                                         cpx<T> (&A)[DFT_LINES], cpx<T> (&B)[DFT_LINES], Load&& load) {
     const int tid = threadIdx.x;
-    TwiddleWalk wa, wb;
+    TwiddleWalk<T> wa, wb;
     wa.start(fa, N, 0);
     wb.start(fb, N, 0);
     X y[DFT_LINES];
@@ -453,46 +345,46 @@ __device__ __forceinline__ void dft_tile(X (*x)[DFT_LINES], const unsigned char*
     }
 }
 
-template <int SRC>
-__global__ __launch_bounds__(256) void k_rowdft_tiled(RowArgs<float> a) {
+template <typename T, int SRC>
+__global__ __launch_bounds__(256) void k_rowdft_tiled(RowArgs<T> a) {
     extern __shared__ __align__(16) unsigned char smem_raw[];    // twiddle table
-    __shared__ __align__(16) float x[DFT_STAGE][DFT_LINES];
+    __shared__ __align__(16) T x[DFT_STAGE][DFT_LINES];
     const int N = a.N, Rs = a.Rs, C = N / 2 + 1, tid = threadIdx.x;
     const int kk0 = DFT_LINES * blockIdx.x, l0 = DFT_FREQS * blockIdx.y + tid;
     load_twiddles(smem_raw, a.tw, N, tid);
     int k[DFT_LINES];
 #pragma unroll
     for (int r = 0; r < DFT_LINES; ++r) k[r] = compact_to_row(min(kk0 + r, 2 * Rs - 1), Rs, N);
-    cpx<float> A[DFT_LINES] = {}, B[DFT_LINES] = {};
-    dft_tile(x, smem_raw, N, Rs, min(l0, C - 1), min(l0 + 256, C - 1), A, B, [&](int s, float (&y)[DFT_LINES]) {
+    cpx<T> A[DFT_LINES] = {}, B[DFT_LINES] = {};
+    dft_tile(x, smem_raw, N, Rs, min(l0, C - 1), min(l0 + 256, C - 1), A, B, [&](int s, T (&y)[DFT_LINES]) {
         const int n = s < Rs ? s : s + N - 2 * Rs;
 #pragma unroll
-        for (int r = 0; r < DFT_LINES; ++r) y[r] = row_source<float, SRC>(a, k[r], n);
+        for (int r = 0; r < DFT_LINES; ++r) y[r] = row_source<T, SRC>(a, k[r], n);
     });
 #pragma unroll
     for (int r = 0; r < DFT_LINES; ++r) {
         if (kk0 + r >= 2 * Rs) break;
-        cpx<float>* out = a.Tm + size_t(kk0 + r) * a.ldT;
+        cpx<T>* out = a.Tm + size_t(kk0 + r) * a.ldT;
         if (l0 < C) out[l0] = A[r];
         if (l0 + 256 < C) out[l0 + 256] = B[r];
     }
 }
 
 // (the row spectra are padded to whole groups of four columns)
-template <int OUT>
-__global__ __launch_bounds__(256) void k_coldft_tiled(ColArgs<float> a) {
+template <typename T, int OUT>
+__global__ __launch_bounds__(256) void k_coldft_tiled(ColArgs<T> a) {
     extern __shared__ __align__(16) unsigned char smem_raw[];    // twiddle table
-    __shared__ __align__(16) cpx<float> x[DFT_STAGE][DFT_LINES];
+    __shared__ __align__(16) cpx<T> x[DFT_STAGE][DFT_LINES];
     const int N = a.N, Rs = a.Rs, C = N / 2 + 1, tid = threadIdx.x;
     const int c0 = DFT_LINES * blockIdx.x, k0 = DFT_FREQS * blockIdx.y + tid;
     load_twiddles(smem_raw, a.tw, N, tid);
-    cpx<float> A[DFT_LINES] = {}, B[DFT_LINES] = {};
-    dft_tile(x, smem_raw, N, Rs, min(k0, N - 1), min(k0 + 256, N - 1), A, B, [&](int s, cpx<float> (&y)[DFT_LINES]) {
-        const cpx<float>* src = a.Tm + size_t(s) * a.ldT + c0;
+    cpx<T> A[DFT_LINES] = {}, B[DFT_LINES] = {};
+    dft_tile(x, smem_raw, N, Rs, min(k0, N - 1), min(k0 + 256, N - 1), A, B, [&](int s, cpx<T> (&y)[DFT_LINES]) {
+        const cpx<T>* src = a.Tm + size_t(s) * a.ldT + c0;
 #pragma unroll
         for (int c = 0; c < DFT_LINES; ++c) y[c] = src[c];
     });
-    const auto store = [&](int col, int k, cpx<float> X) {
+    const auto store = [&](int col, int k, cpx<T> X) {
         if (col >= C || k >= N) return;
         if constexpr (OUT == OUT_COLMAJOR_SHIFT) a.S[size_t(col) * a.ldS + (k < N / 2 ? k + N / 2 : k - N / 2)] = X;
         else a.S[size_t(k) * C + col] = X;
@@ -505,9 +397,8 @@ __global__ __launch_bounds__(256) void k_coldft_tiled(ColArgs<float> a) {
 }
 
 // ---------------------------------------------------------------------------
-// even N that none of these covers (in double up to 64, or beyond half the largest workgroup transform and no
-// power of two; in float no power of two whose twiddle table LDS does not hold beside the others'): as
-// above, one output at a time.
+// even N whose twiddle table is too large for that (in double beyond 4096, in float beyond 8192): as above, one output
+// at a time.
 // ---------------------------------------------------------------------------
 template <typename T, int SRC>
 __global__ __launch_bounds__(256) void k_rowdft_generic(RowArgs<T> a) {
