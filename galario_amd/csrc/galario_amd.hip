@@ -102,6 +102,15 @@ void check_dev_inputs(const T* I, int nd, const T* u, const T* v, bool obs, cons
     if (nd > 0 && (!u || !v)) invalid("check input", "null u or v pointer");
     if (nd > 0 && obs && (!re || !im || !w)) invalid("check input", "null observed-visibility or weight pointer");
 }
+// Arrays of a host-array call, likewise: `input` is the profile or the image, `out` the result.  (Small arrays are read and
+// written by the calling thread itself, and the sample kernel takes what it is given.)
+template <typename T>
+void check_host_arrays(const T* input, const char* what, int nd, const T* u, const T* v, bool obs, const T* re,
+                       const T* im, const T* w, const T* out) {
+    if (!input) invalid("check input", std::string("null ") + what + " pointer");
+    check_dev_inputs(input, nd, u, v, obs, re, im, w);
+    if ((obs || nd > 0) && !out) invalid("check input", obs ? "null chi2 pointer" : "null visibility pointer");
+}
 
 // ------------------------------------------------------------------ memory
 struct DevBuf {
@@ -879,6 +888,7 @@ int sample_profile_host(int nr, const T* I, T Rmin, T dR, T dxy, int nxy, T inc,
         check_nd(nd);
         ProfileSetup<T> ps = setup_profile<T>(nr, Rmin, dR, dxy, nxy, inc, check_central);
         SampleSetup<T> ss = setup_sample<T>(PA, dRA, dDec);
+        check_host_arrays<T>(I, "intensity", nd, u, v, false, nullptr, nullptr, nullptr, vis);
         Workspace& w = workspace(nullptr, true);
         hipStream_t s = w.own;
         Inputs in(w, s, Inputs::room(sizeof(T) * size_t(nr)) + 2 * Inputs::room(sizeof(T) * size_t(nd)));
@@ -899,6 +909,7 @@ int chi2_profile_host(int nr, const T* I, T Rmin, T dR, T dxy, int nxy, T inc, T
         check_nd(nd);
         ProfileSetup<T> ps = setup_profile<T>(nr, Rmin, dR, dxy, nxy, inc, check_central);
         SampleSetup<T> ss = setup_sample<T>(PA, dRA, dDec);
+        check_host_arrays<T>(I, "intensity", nd, u, v, true, re, im, wt, chi2);
         Workspace& w = workspace(nullptr, true);
         hipStream_t s = w.own;
         Inputs in(w, s, Inputs::room(sizeof(T) * size_t(nr)) + 5 * Inputs::room(sizeof(T) * size_t(nd)));
@@ -921,6 +932,7 @@ int sample_image_host(int nx, int ny, const T* image, T v_origin, T dRA, T dDec,
         check_nd(nd);
         check_input_xy(nx, ny);
         SampleSetup<T> ss = setup_sample<T>(PA, dRA, dDec);
+        check_host_arrays<T>(image, "image", nd, u, v, false, nullptr, nullptr, nullptr, vis);
         Workspace& w = workspace(nullptr, true);
         hipStream_t s = w.own;
         const int N = nx, C = N / 2 + 1;
@@ -946,6 +958,7 @@ int chi2_image_host(int nx, int ny, const T* image, T v_origin, T dRA, T dDec, T
         check_nd(nd);
         check_input_xy(nx, ny);
         SampleSetup<T> ss = setup_sample<T>(PA, dRA, dDec);
+        check_host_arrays<T>(image, "image", nd, u, v, true, re, im, wt, chi2);
         Workspace& w = workspace(nullptr, true);
         hipStream_t s = w.own;
         const int N = nx, C = N / 2 + 1;
