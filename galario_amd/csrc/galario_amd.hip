@@ -857,18 +857,28 @@ struct Inputs {
     unsigned* flag() const { return reinterpret_cast<unsigned*>(w.h_scal + 1); }
 };
 
-// Synchronise the own stream and raise if a point fell outside the grid.
-void finish_host_call(Workspace& w, hipStream_t s) {
+// Wait for the own stream; then the results are in place.
+void wait_host_call(Workspace& w, hipStream_t s) {
     t_timer.end_call(s);
     HC(hipStreamSynchronize(s));
     w.stage_busy = false;
+}
+
+// Raise if a point of the finished call fell outside the grid.
+void check_outside(const Workspace& w) {
     if (*reinterpret_cast<volatile unsigned*>(w.h_scal + 1))
         invalid("interpolate",
                 "at least one (u, v) point falls outside the Fourier grid (|u|/duv must not exceed ncol-1 and "
                 "nrow/2 + v/duv must lie in [0, nrow-1]); increase nxy or reduce dxy");
 }
 
-// Visibilities into the host array vis: up to STAGE_ARRAY bytes are written to pinned memory by the kernel.
+void finish_host_call(Workspace& w, hipStream_t s) {
+    wait_host_call(w, s);
+    check_outside(w);
+}
+
+// Visibilities into the host array vis: up to STAGE_ARRAY bytes are written to pinned memory by the kernel.  They
+// reach vis whether or not a point lies outside the grid (its own is NaN).
 template <typename T>
 void launch_vis_host(Inputs& in, hipStream_t s, const SampleArgs<T>& sa, cpx<T>* vis) {
     const size_t n = size_t(sa.nd), bytes = n * sizeof(cpx<T>);
@@ -876,8 +886,9 @@ void launch_vis_host(Inputs& in, hipStream_t s, const SampleArgs<T>& sa, cpx<T>*
     cpx<T>* d = pinned ? reinterpret_cast<cpx<T>*>(in.w.h_out.get(bytes)) : in.w.out.template get<cpx<T>>(n);
     launch_vis(s, sa, d);
     if (!pinned) download(vis, d, n, s);
-    finish_host_call(in.w, s);
+    wait_host_call(in.w, s);
     if (pinned && n) std::memcpy(vis, d, bytes);
+    check_outside(in.w);
 }
 
 // ------------------------------------------------------------------ main functions (host pointers)
