@@ -1071,7 +1071,8 @@ __device__ __forceinline__ cpx<P> sample_point_sym2(const SampleArgs<T>& a, cons
     P s = P(0), c = P(1);
     if (std::is_same<P, double>::value || sc.phase) phase_factor(sc, p.urot, p.vrot, &s, &c);
     const P V0 = sym_amplitude(y, p.q, p.t);
-    return cpx<P>{V0 * c, V0 * s};
+    // (plus zero: without an offset the imaginary part of a negative V0 is +0, its angle +pi)
+    return cpx<P>{V0 * c, ffma(V0, s, P(0))};
 }
 
 // Visibility of a point on the real path; NaN and oob outside the grid or the extent.
