@@ -1085,7 +1085,8 @@ __device__ __forceinline__ cpx<T> sample_point_sym(const SampleArgs<T>& a, T u0,
 }
 
 // chi2 term w |V - O|^2 of a point.  In double from w itself (galario multiplies the residual by sqrt(w),
-// src/galario.cpp:1453-1461: NaN for a negative weight, which is kept); in float in galario's order.
+// src/galario.cpp:1453-1461: NaN for a negative weight, which is kept), one factor of the residual at a time: no step
+// leaves the range of a double where the term itself is within it.  In float in galario's order.
 template <typename P>
 __device__ __forceinline__ P weight_factor(P w) {
     if constexpr (std::is_same<P, double>::value) return w < P(0) ? P(NAN) : w;
@@ -1094,7 +1095,7 @@ __device__ __forceinline__ P weight_factor(P w) {
 template <typename P>
 __device__ __forceinline__ double chi2_term(P wf, P dre, P dim) {
     if constexpr (std::is_same<P, double>::value) {
-        return wf * ffma(dre, dre, dim * dim);
+        return ffma(wf * dre, dre, (wf * dim) * dim);
     } else {
         const P cr = dre * wf, ci = dim * wf;
         return double(cr) * cr + double(ci) * ci;
