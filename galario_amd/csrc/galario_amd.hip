@@ -1398,6 +1398,7 @@ struct BatchPlan : BatchPlanBase {
         int ppt = 1;                   // 256-point blocks per sample workgroup (forward)
         int win = GWIN;                // LDS window cells of the gradient sample kernel
         bool tile_fixed = false;       // ppt / win set by the caller: the autotuner keeps them
+        bool chunk_fixed = false;      // chunk set by the caller: every grid takes it as it is
         hipGraphExec_t exec = nullptr;
     };
     std::map<std::pair<int, int>, Exec> runs;   // (nwalkers, mode)
@@ -1530,13 +1531,15 @@ void launch_sample_grad(int win, int nb, int nw, hipStream_t s, const SampleArgs
 // Launch shape of one batched evaluation.
 struct BatchShape {
     int chunk, kw, ppt, win;
+    bool by_grid;            // a grid takes fewer walkers than chunk where group_chunk says so
 };
 
 // Walkers of a grid processed together in the forward form when a plan has several grids: at most `chunk`, and no more
-// than whose half spectra the 256 MB MALL about holds (a power of two, at least 8), since the samples then
-// read them from there.  256 walkers, nxy = 2048 and 1e6 points: 1.48 ms with 32, 1.54 with 128; nxy = 1024 and
-// 2e5 points, whose 128 spectra fit: 0.39 with 128, 0.53 with 32.  (With one grid the timed choice is that grid's own; the
-// gradient form, bound by its atomics, takes the largest chunk.)
+// than whose half spectra come to 288 MB (a power of two, at least 8), since the samples then read most of them from
+// the 256 MB MALL.  256 walkers, nxy = 2048 and 1e6 points: 1.48 ms with 32, 1.54 with 128; nxy = 1024 and
+// 2e5 points, whose 128 spectra are 274 MB: 0.39 with 128, 0.53 with 32.  64 walkers, nxy = 4096 and 1e6 points beside
+// nxy = 512: 0.90 with 8 on the larger grid, 0.96 with 64; 5000 points: 0.53 and 0.58.  (With one grid the timed choice is that grid's own; the gradient form, bound by its atomics,
+// takes the largest chunk.)
 template <typename T>
 int group_chunk(const BatchPlan<T>& P, const BatchGroup<T>& G, int chunk, bool grad) {
     if (grad || P.groups.size() < 2) return chunk;
@@ -1544,6 +1547,14 @@ int group_chunk(const BatchPlan<T>& P, const BatchGroup<T>& G, int chunk, bool g
     int c = 8;
     while (size_t(2 * c) * bytes <= (size_t(288) << 20)) c *= 2;
     return std::min(c, chunk);
+}
+
+// Largest chunk that any grid of the plan takes: more slots would hold nothing, and larger chunks all launch the same.
+template <typename T>
+int largest_chunk(const BatchPlan<T>& P, bool grad, int W) {
+    int c = 1;
+    for (const BatchGroup<T>& G : P.groups) c = std::max(c, group_chunk(P, G, P.max_chunk(grad, W), grad));
+    return c;
 }
 
 template <typename T>
@@ -1567,7 +1578,7 @@ void batch_enqueue(BatchPlan<T>& P, hipStream_t s, int W, const BatchShape& sh, 
     BatchPtrs<T> b = batch_ptrs(P, grad);
     unsigned* flag = static_cast<unsigned*>(P.flag.p);
     for (const BatchGroup<T>& G : P.groups) {
-        const int gchunk = group_chunk(P, G, chunk, grad);
+        const int gchunk = sh.by_grid ? group_chunk(P, G, chunk, grad) : chunk;
         for (int w0 = 0; w0 < W; w0 += gchunk) {
             const int nw = std::min(gchunk, W - w0);
             b.w0 = w0;
@@ -1778,18 +1789,18 @@ float batch_time(BatchPlan<T>& P, hipStream_t s, int W, const BatchShape& sh, in
 // Launch shape for W walkers, by timing eager evaluations on the caller's
 // stream, one dimension at a time from (4 walkers per sample workgroup, one
 // 256-point block per workgroup, 3072-cell gradient window): the chunk size
-// (powers of two and W itself, within the slot budget); forward: the walkers
+// (powers of two and largest_chunk); forward: the walkers
 // per sample workgroup (1, 2, 4, 8), then the point blocks per workgroup
 // (1, 2); gradient: the LDS window (2048, 3072, 4096 cells).  Point blocks and
 // window set by the caller (tile_fixed) are kept.
 template <typename T>
 void batch_tune(BatchPlan<T>& P, hipStream_t s, int W, int mode, typename BatchPlan<T>::Exec& run) {
     const bool grad = mode & MODE_GRAD;
-    const int cmax = P.max_chunk(grad, W);
+    const int cmax = largest_chunk(P, grad, W);
     std::vector<int> cand{cmax};                     // largest first
     for (int c = cmax - 1; c > 0; --c)
         if (!(c & (c - 1))) cand.push_back(c);
-    BatchShape best{cand.front(), 4, run.tile_fixed ? run.ppt : 1, run.tile_fixed ? run.win : GWIN};
+    BatchShape best{cand.front(), 4, run.tile_fixed ? run.ppt : 1, run.tile_fixed ? run.win : GWIN, true};
     float tbest = 0.f;
     for (int c : cand) {
         BatchShape t = best;
@@ -1836,7 +1847,7 @@ void batch_tune(BatchPlan<T>& P, hipStream_t s, int W, int mode, typename BatchP
 
 template <typename T>
 BatchShape shape_of(const typename BatchPlan<T>::Exec& run) {
-    return BatchShape{run.chunk, run.kw, run.ppt, run.win};
+    return BatchShape{run.chunk, run.kw, run.ppt, run.win, !run.chunk_fixed};
 }
 
 // geom of type G: T, or double with MODE_F64_PHASE (float plans only).
@@ -2258,6 +2269,7 @@ int galario_batch_set_chunk(void* plan, int nwalkers, int mode, int chunk, int w
             if (run.exec) (void)hipGraphExecDestroy(run.exec);
             run.exec = nullptr;
             run.chunk = chunk;
+            run.chunk_fixed = true;
             run.kw = walkers_per_sample;
         };
         if (b->prec == 8) set(*static_cast<BatchPlan<double>*>(b));

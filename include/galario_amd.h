@@ -357,13 +357,15 @@ int galario_batch_chi2_profile_grad_f32x(void *plan, void *stream, int nwalkers,
 #define GALARIO_BATCH_MODE_GRAD 1       /* the _grad calls */
 #define GALARIO_BATCH_MODE_F64_PHASE 2  /* the _f32x calls (float plans) */
 /* The launch shape picked for (nwalkers, mode): chunk size (0 before the
- * first call) and walkers per sample workgroup (the forward sample reads each
- * dataset point once for that many walkers; 1 with the gradient), and
- * whether its graph is captured.  Any pointer may be null. */
+ * first call; with several grids the largest that a grid takes, larger grids
+ * fewer, unless galario_batch_set_chunk set it) and walkers per sample
+ * workgroup (the forward sample reads each dataset point once for that many
+ * walkers; 1 with the gradient), and whether its graph is captured.  Any
+ * pointer may be null. */
 int galario_batch_info(void *plan, int nwalkers, int mode, int *chunk, int *walkers_per_sample,
                        int *graph_ready);
-/* Overrides the timed choice for (nwalkers, mode): chunk size and walkers
- * per sample workgroup (1, 2, 4 or 8). */
+/* Overrides the timed choice for (nwalkers, mode): chunk size (every grid
+ * takes it as it is) and walkers per sample workgroup (1, 2, 4 or 8). */
 int galario_batch_set_chunk(void *plan, int nwalkers, int mode, int chunk, int walkers_per_sample);
 /* The tile of (nwalkers, mode)'s sample kernel, chosen with the chunk
  * (0 before the first call): forward -- point_blocks, the 256-point blocks
