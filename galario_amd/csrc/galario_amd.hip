@@ -788,12 +788,14 @@ void download(X* h, const X* d, size_t n, hipStream_t s) {
     if (n) HC(hipMemcpyAsync(h, d, n * sizeof(X), hipMemcpyDeviceToHost, s));
 }
 
-// Inputs and results of a host-array call.  Arrays of up to STAGE_ARRAY bytes (STAGE_BYTES in all) are packed into
+// Inputs and results of a host-array call.  Arrays below STAGE_ARRAY bytes (STAGE_BYTES in all) are packed into
 // pinned memory, which a small kernel copies to the device, STAGE_PART bytes at a time so that the copy of
 // one part runs while the next is packed: a call's six copies of a few KB cost 6 to 8 us of host
 // time each, the packed copy one launch (2013 points at nxy = 512: 78 -> 36 us a call; 40000 points
 // 127 -> 86; 2e5 points 325 -> 292).  Larger arrays go by a copy each, whose rate a copy through pinned
-// memory by one host thread does not reach (8 MB: 241 against 400 us).  The result and the out-of-grid
+// memory by one host thread does not reach (8 MB: 241 against 400 us).  The line lies at 2 MiB, where the copy of
+// pageable memory itself gets faster: chi2 of arrays of 2 MiB - 8 bytes takes 359 us packed and 370 by copies, of 2 MiB 358
+// and 332; an image of 2 MiB 151 and 127.  The result and the out-of-grid
 // flag are written to pinned memory by the kernels themselves.
 constexpr size_t STAGE_BYTES = size_t(8) << 20, STAGE_ARRAY = size_t(2) << 20, STAGE_PART = size_t(512) << 10;
 
@@ -819,7 +821,7 @@ struct Inputs {
     template <class X>
     const X* add(DevBuf& b, const X* h, size_t n) {
         const size_t bytes = n * sizeof(X);
-        if (bytes > STAGE_ARRAY || off + room(bytes) > cap) return upload(b, h, n, s);
+        if (bytes >= STAGE_ARRAY || off + room(bytes) > cap) return upload(b, h, n, s);
         char* to = w.h_in.p + off;
         const X* d = reinterpret_cast<const X*>(dev + off);
         if (n) std::memcpy(to, h, bytes);
