@@ -794,7 +794,7 @@ void download(X* h, const X* d, size_t n, hipStream_t s) {
 // time each, the packed copy one launch (2013 points at nxy = 512: 78 -> 36 us a call; 40000 points
 // 127 -> 86; 2e5 points 325 -> 292).  Larger arrays go by a copy each, whose rate a copy through pinned
 // memory by one host thread does not reach (8 MB: 241 against 400 us).  The line lies at 2 MiB, where the copy of
-// pageable memory itself gets faster: chi2 of arrays of 2 MiB - 8 bytes takes 359 us packed and 370 by copies, of 2 MiB 358
+// pageable memory itself gets faster: chi2 of arrays of 250000 doubles takes 343 us packed and 362 by copies, of 262144, 358
 // and 332; an image of 2 MiB 151 and 127.  The result and the out-of-grid
 // flag are written to pinned memory by the kernels themselves.
 constexpr size_t STAGE_BYTES = size_t(8) << 20, STAGE_ARRAY = size_t(2) << 20, STAGE_PART = size_t(512) << 10;
@@ -1540,8 +1540,8 @@ struct BatchShape {
 // than whose half spectra come to 288 MB (a power of two, at least 8), since the samples then read most of them from
 // the 256 MB MALL.  256 walkers, nxy = 2048 and 1e6 points: 1.48 ms with 32, 1.54 with 128; nxy = 1024 and
 // 2e5 points, whose 128 spectra are 274 MB: 0.39 with 128, 0.53 with 32.  64 walkers, nxy = 4096 and 1e6 points beside
-// nxy = 512: 0.90 with 8 on the larger grid, 0.96 with 64; 5000 points: 0.53 and 0.58.  (With one grid the timed choice is that grid's own; the gradient form, bound by its atomics,
-// takes the largest chunk.)
+// nxy = 512: 0.90 with 8 on the larger grid, 0.96 with 64; 5000 points: 0.53 and 0.58.  (With one grid the timed
+// choice is that grid's own; the gradient form, bound by its atomics, takes the largest chunk.)
 template <typename T>
 int group_chunk(const BatchPlan<T>& P, const BatchGroup<T>& G, int chunk, bool grad) {
     if (grad || P.groups.size() < 2) return chunk;
@@ -1616,7 +1616,6 @@ void batch_enqueue(BatchPlan<T>& P, hipStream_t s, int W, const BatchShape& sh, 
                 a.ldH = g.ldH;
                 a.nrow = G.N;
                 a.ncol = g.C;
-                a.v_origin = T(1);
                 a.duv = d.duv;
                 a.inv_duv = T(1) / d.duv;
                 a.nd = d.nd;

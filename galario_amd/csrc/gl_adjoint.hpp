@@ -79,7 +79,7 @@ __device__ __forceinline__ double xor_sign(double x, double s) {   // x with its
     return __hiloint2double(__double2hiint(x) ^ (__double2hiint(s) & int(0x80000000u)), __double2loint(x));
 }
 
-// The same at a byte offset below 2^32 from a uniform base (Hh holds at most 2^29 bytes).
+// The same at a byte offset below 2^32 from a uniform base (Hh holds less than 2^30 bytes).
 __device__ __forceinline__ void atomic_add_at(double* base, unsigned bytes, double v) {
     atomic_add_f64(reinterpret_cast<double*>(reinterpret_cast<char*>(base) + size_t(bytes)), v);
 }
@@ -214,7 +214,7 @@ __device__ __forceinline__ void sample_grad_sym_body(const SampleArgs<T>& a, con
     const int pmax = 0xFFFF - int(min(h0 & 0xFFFFu, h1 & 0xFFFFu)), mmax = 0xFFFF - int(min(h0 >> 16, h1 >> 16));
     const bool any = pmin <= pmax;                   // (no live point: 0xFFFF and 0)
     const int wp = pmax - pmin + 1, w2 = 2 * (mmax - mmin + 1);
-    const bool use_win = any && wp * w2 <= WIN;      // (wp, w2 <= 2^14, no overflow)
+    const bool use_win = any && wp * w2 <= WIN;      // (wp <= 2^12 + 1, w2 <= 2^14 + 2: no overflow)
     const int nwin = use_win ? wp * w2 : 0;          // even
     const int nclear = use_win ? nwin : GPT == 1 && g.direct ? GHOT * GHOT : WIN;
     for (int j = 2 * tid; j < nclear; j += 512)
@@ -414,8 +414,11 @@ constexpr int GPT_SINGLE = 1, GPT_BATCH = 2;
 constexpr size_t GRAD_FEW_WORKGROUPS = 8192;
 // Launches of at most this many workgroups add their sparse points straight to Hh: all of them are resident at once, so
 // the launch takes one workgroup's latency, to which the line table's building and flush add 2 to 4 us, while the
-// atomics' rate does not bind yet.  nxy = 4096, direct against table: 8000 points 4.9 / 8.4 us, 64000 7.1 / 8.4,
-// 128000 11.1 / 10.2, 256000 14.4 / 13.0; nxy = 1024: 8000 4.4 / 9.4, 128000 6.2 / 9.4.
+// atomics' rate does not bind yet.  The kernel, direct against table: nxy = 4096, 8000 points 4.9 / 8.4 us, 64000 7.1 / 8.4,
+// 128000 11.1 / 10.2, 256000 14.4 / 13.0; nxy = 1024, 8000 4.4 / 9.4, 128000 6.2 / 9.4.  The gradient call at 131000
+// points: nxy = 1024 32.3 / 34.6 us, 2048 37.0 / 38.9, 4096 56.1 / 55.2, 8192 128.1 / 130.3.  (At 4096 the two meet at
+// 90000 points, 350 workgroups, and the table would save 0.9 us of the call at 512; a lower line would cost the other
+// sizes 2 us.)
 constexpr int GRAD_DIRECT_BLOCKS = 512;
 template <typename T>
 __global__ __launch_bounds__(256) void k_sample_grad_sym(SampleArgs<T> a, GradArgs<T> g) {

@@ -22,15 +22,13 @@ namespace gl {
 template <typename T>
 struct WalkerPrm {
     T cos_inc;
-    int rotate;
     T cosPA, sinPA;
-    int phase;
-    T dRA2, dDec2;       // 2 pi dRArot, 2 pi dDecrot
-    T dRAt, dDect;       // dRArot, dDecrot (the phase in turns)
+    int phase;           // float: whether there is an offset
+    T dRA2, dDec2;       // float: 2 pi dRArot, 2 pi dDecrot
+    T dRAt, dDect;       // double: dRArot, dDecrot (the phase in turns)
     double tan_inc;
     // the same rotation and phase scalars in double (the FP32-bulk form's FP64 per-point arithmetic)
-    double cosPAd, sinPAd, dRA2d, dDec2d, dRAtd, dDectd;
-    int phased;
+    double cosPAd, sinPAd, dRAtd, dDectd;
 };
 
 // geom: [W][4] = inc, PA, dRA, dDec, of type G (T, or double for the FP32-bulk form with FP64
@@ -48,13 +46,11 @@ __global__ __launch_bounds__(256) void k_batch_setup(int W, const G* __restrict_
         p.tan_inc = tan(double(geom[4 * i]));
         T dRArot, dDecrot;
         if (PA == T(0)) {
-            p.rotate = 0;
             p.cosPA = T(1);
             p.sinPA = T(0);
             dRArot = dRA;
             dDecrot = dDec;
         } else {
-            p.rotate = 1;
             p.cosPA = T(cos(double(PA)));
             p.sinPA = T(sin(double(PA)));
             dRArot = dRA * p.cosPA - dDec * p.sinPA;
@@ -75,9 +71,6 @@ __global__ __launch_bounds__(256) void k_batch_setup(int W, const G* __restrict_
             dRArotd = dRAd * p.cosPAd - dDecd * p.sinPAd;
             dDecrotd = dRAd * p.sinPAd + dDecd * p.cosPAd;
         }
-        p.phased = !(dRArotd == 0.0 && dDecrotd == 0.0);
-        p.dRA2d = dRArotd * (2. * M_PI);
-        p.dDec2d = dDecrotd * (2. * M_PI);
         p.dRAtd = dRArotd;
         p.dDectd = dDecrotd;
         wp[i] = p;
@@ -143,7 +136,6 @@ template <typename T>
 __device__ __forceinline__ void walker_sample_args(SampleArgs<T>& a, const BatchPtrs<T>& b, int slot, int w) {
     const WalkerPrm<T> p = b.wp[w];
     a.H = b.H + slot * b.sH;
-    a.rotate = p.rotate;
     a.cosPA = p.cosPA;
     a.sinPA = p.sinPA;
     a.phase = p.phase;
@@ -162,16 +154,11 @@ __device__ __forceinline__ SampleArgs<double> walker_scalars_f64(const SampleArg
     SampleArgs<double> sc{};
     sc.nrow = a.nrow;
     sc.ncol = a.ncol;
-    sc.v_origin = double(a.v_origin);
     sc.duv = a.duv_d;
     sc.inv_duv = a.inv_duv_d;
     sc.ext2 = a.ext2;
-    sc.rotate = p.rotate;
     sc.cosPA = p.cosPAd;
     sc.sinPA = p.sinPAd;
-    sc.phase = p.phased;
-    sc.dRA2 = p.dRA2d;
-    sc.dDec2 = p.dDec2d;
     sc.dRAt = p.dRAtd;
     sc.dDect = p.dDectd;
     return sc;

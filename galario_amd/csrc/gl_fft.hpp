@@ -383,8 +383,8 @@ struct ResidueFft {
     // few bank conflicts more, but every exchange address is a per-lane base plus a constant (positions
     // base + r, base + 8 r and lane + 64 r go to slots base' + r, base' + 9 r and lane' + 72 r), so the
     // offsets fold into the LDS instructions: the column pass's code has 33 fewer VALU and 16 fewer LDS
-    // instructions, and its workgroups fit on a CU as before (its LDS is sized by the output transpose).  The adjoint column pass
-    // keeps the 512-slot form, where 576 slots would cost a workgroup per CU.
+    // instructions, and its workgroups fit on a CU as before (its LDS is sized by the output transpose).  The
+    // adjoint column pass keeps the 512-slot form, where 576 slots would cost a workgroup per CU.
     static __device__ __forceinline__ int slot(int i) { return PAD ? i + (i >> 3) : i ^ ((i >> 3) & 15); }
 
     template <int P, int PART>

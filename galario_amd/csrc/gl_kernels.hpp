@@ -9,9 +9,11 @@
 //         k (the reference's fftshift_axis0 folded into the stores).
 //         The four interpolation corners are then two 32-byte pairs.
 //
-// All stages that restate galario arithmetic (sweep, central pixel,
-// interpolation, phase, chi2 terms) are compiled without FMA contraction so
-// they round exactly as the reference's -std=c++11 x86-64 build.
+// The stages that restate galario arithmetic (sweep, central pixel, and on
+// the complex spectrum and in float interpolation, phase and chi2 terms) are
+// compiled without FMA contraction so they round exactly as the reference's
+// -std=c++11 x86-64 build.  In double on the real spectrum the sample point
+// has a shorter order with explicit fused operations (sym_position and below).
 #pragma once
 
 #include <type_traits>
@@ -946,16 +948,16 @@ __device__ __forceinline__ cpx<T> sample_point(const SampleArgs<T>& a, T u0, T v
 //
 // Storage and arithmetic may differ: the spectrum H is read from `a` (type T)
 // while the position, interpolation and phase use the scalars of `sc` and
-// arithmetic in P.  P = T (sc = a) is galario's arithmetic in that precision;
+// arithmetic in P.  P = T (sc = a) is that precision throughout (float: galario's order);
 // T = float, P = double is the FP32-bulk form with FP64 per-point arithmetic.
 //
-// The batched sample kernels issue vector instructions at 60 to 85% of the rate the chip can (nxy = 4096 and 2048;
-// 130 instructions per walker and 64 points became 105: 256 walkers x 3 datasets 2.58 to 2.11 ms), so the forms below are the ones with few instructions and no branches (a branch also
-// keeps the loads of one point behind the arithmetic of another): without a rotation the scalars are
-// cos = 1, sin = 0 (no selection per point), without offsets the phase factor of 0 is computed; the
-// real path's v_origin is 1; the extent is checked on the unrotated radius, once per point for all
+// The batched sample kernels issue vector instructions at 60 to 85% of the rate the chip can (nxy = 4096 and
+// 2048; 130 instructions per walker and 64 points became 106: 256 walkers x 3 datasets 2.58 to 2.11 ms), so the
+// forms below are the ones with few instructions and no branches (a branch also keeps the loads of one point
+// behind the arithmetic of another): without a rotation the scalars are cos = 1, sin = 0 (no selection per
+// point), without offsets the phase factor of 0 is computed; the real path's v_origin is 1; the extent is checked on the unrotated radius, once per point for all
 // walkers; the fraction of the position comes from one instruction; corners are 32-bit byte
-// offsets from H (H holds at most 2^28 bytes); in double the bilinear forms are nested fused products.
+// offsets from H (H holds less than 2^29 bytes); in double the bilinear forms are nested fused products.
 // Every kernel samples through these functions, so one point gives the same bits in all of them.
 template <typename P>
 struct SymPoint {
